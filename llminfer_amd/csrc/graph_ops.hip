@@ -10,11 +10,23 @@
 //    bits; SiLU goes through the same correctly rounded helper as the
 //    projections' epilogue.
 //  * linearF16 keeps the reference's arithmetic: each output is one fp32
-//    fma chain over k = 0 .. K-1 in order, then storeLinear. A workgroup of
-//    256 lanes serves 256 output columns and up to 8 rows; 64-wide k chunks
-//    of the 256 weight rows are staged in LDS (rows padded by 16 bytes, so
-//    lane c's 16-byte reads of its own row meet no bank conflicts) and a
-//    lane runs its rows' chains side by side.
+//    fma chain over k = 0 .. K-1 in order, then storeLinear. The chain runs on
+//    v_mfma_f32_16x16x4_f32, which adds its four products to the sum in k
+//    order, each step rounded as an fma (checked bit for bit against the
+//    scalar chain): 3.4 ns a k value for a 16 x 16 tile at any depth of
+//    dependence, where a lane's fma chain takes 3.9. That chain bounds a tile
+//    (31 us at K = 9216) and 157 TFLOP/s the chip, so every tile of a step
+//    must keep its matrix core fed: waves that compute touch LDS and the
+//    matrix core only, other waves load the rows (16 bytes a lane, 256 a row),
+//    and stage them as MFMA operands: lane group g = lane / 16 of an operand
+//    holds the halves k = 4 s + g of its row, so the halves (g, g + 4) of
+//    eight consecutive ones go as a dword to group g's lane, and a 16-byte
+//    read gives a lane its values of eight steps. Three buffers: the first
+//    chunk of the next step is read before the barrier. The three projections
+//    of an MLP (2560 -> 9216 -> 2560) for 93 rows 2751 -> 187 us, for one row
+//    2740 -> 97 us, against a lane-per-column fma kernel; what is left above
+//    the chains is the conversions (a matrix core's fp32 products and the VALU
+//    do not overlap) and the staging.
 #include "exact_fp.hpp"
 #include "hip_common.hpp"
 #include "kernels.hpp"
@@ -78,69 +90,183 @@ __global__ __launch_bounds__(256) void copy_view_kernel(const uint16_t *__restri
   out[i] = src[offset];
 }
 
-constexpr unsigned kF16Cols = 256, kF16Rows = 8, kF16Chunk = 64;
-constexpr unsigned kF16Pitch = kF16Chunk + 8; // halves per staged weight row
+// ------------------------------------------------------------- linearF16
 
-__global__ __launch_bounds__(kF16Cols) void linear_f16_kernel(
-    const uint16_t *__restrict__ in, const uint16_t *__restrict__ w, void *out, const void *aux,
-    const float *bias, LinearParams p) {
-  __shared__ __align__(16) uint16_t sW[kF16Cols * kF16Pitch];
-  __shared__ __align__(16) float sIn[kF16Rows][kF16Chunk];
-  const unsigned t = threadIdx.x;
-  const unsigned col0 = blockIdx.x * kF16Cols, row0 = blockIdx.y * kF16Rows;
-  const unsigned nr = min(kF16Rows, p.tokens - row0);
-  float acc[kF16Rows];
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+// Eight consecutive halves of a row from k. kVec: rows start 16-byte aligned
+// and hold whole pieces of eight; past the end the last piece again (in
+// bounds; zeroed where it is used, so that nothing waits for the load before
+// then). Else one half at a time, zeros past the end.
+template <bool kVec>
+__device__ __forceinline__ uint4_t load_halves8(const uint16_t *__restrict__ row, unsigned k,
+                                                unsigned width) {
+  if constexpr (kVec)
+    return *reinterpret_cast<const uint4_t *>(row + min(k, width - 8));
+  uint4_t v;
 #pragma unroll
-  for (unsigned r = 0; r < kF16Rows; ++r)
-    acc[r] = 0.0f;
-  for (unsigned base = 0; base < p.inputWidth; base += kF16Chunk) {
-    __syncthreads(); // the previous chunk is consumed
-    // Weight rows col0 .. col0+255, halves base .. base+63 (zero past the
-    // ends): 8 threads per row, 8 halves each, 8 passes.
-    for (unsigned e = t; e < kF16Cols * (kF16Chunk / 8); e += kF16Cols) {
-      const unsigned c = e / (kF16Chunk / 8), k8 = (e % (kF16Chunk / 8)) * 8;
-      const unsigned col = col0 + c;
-      uint16_t v[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const unsigned k = base + k8 + j;
-        v[j] = col < p.rowCount && k < p.inputWidth ? w[(size_t)col * p.inputWidth + k] : 0;
-      }
-      uint4_t packed;
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        packed[j] = (uint32_t)v[2 * j] | ((uint32_t)v[2 * j + 1] << 16);
-      *reinterpret_cast<uint4_t *>(&sW[c * kF16Pitch + k8]) = packed;
-    }
-    for (unsigned e = t; e < kF16Rows * kF16Chunk; e += kF16Cols) {
-      const unsigned r = e / kF16Chunk, k = base + e % kF16Chunk;
-      sIn[r][e % kF16Chunk] =
-          r < nr && k < p.inputWidth ? h2f(in[(size_t)(row0 + r) * p.inputWidth + k]) : 0.0f;
-    }
-    __syncthreads();
-#pragma unroll 2
-    for (unsigned k8 = 0; k8 < kF16Chunk; k8 += 8) {
-      const uint4_t wv = *reinterpret_cast<const uint4_t *>(&sW[t * kF16Pitch + k8]);
-      float wf[8];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        wf[2 * j] = h2f((uint16_t)(wv[j] & 0xFFFFu));
-        wf[2 * j + 1] = h2f((uint16_t)(wv[j] >> 16));
-      }
-#pragma unroll
-      for (unsigned r = 0; r < kF16Rows; ++r)
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          acc[r] = __builtin_fmaf(sIn[r][k8 + j], wf[j], acc[r]);
-    }
+  for (unsigned e = 0; e < 4; ++e) {
+    const unsigned k0 = k + 2 * e;
+    const uint32_t lo = k0 < width ? row[k0] : 0, hi = k0 + 1 < width ? row[k0 + 1] : 0;
+    v[e] = lo | (hi << 16);
   }
-  const unsigned col = col0 + t;
+  return v;
+}
+
+constexpr unsigned kF16Tile = 16, kF16Chunk = 32, kF16Chunks = 4;
+constexpr unsigned kF16Step = kF16Chunk * kF16Chunks;      // k values a step
+constexpr unsigned kF16ChunkBytes = 1024 + 64;             // 64 lanes x 16 B, and a pad
+constexpr unsigned kF16TileBytes = kF16Chunks * kF16ChunkBytes;
+constexpr unsigned kF16Buffers = 3, kF16FewTiles = 512;
+
+// kRT x kCT tiles a workgroup, a wave a tile, and kLoaders staging waves whose
+// loads run kDepth steps ahead of their staging.
+template <int kRT, int kCT, int kLoaders, int kDepth, bool kVec>
+__global__ __launch_bounds__(64 * (kRT * kCT + kLoaders)) void linear_f16_kernel(
+    const uint16_t *__restrict__ in, const uint16_t *__restrict__ w, void *out, const void *aux,
+    const float *bias, LinearParams p, unsigned rowBlocks) {
+  constexpr unsigned kThreads = 64 * kLoaders;
+  constexpr unsigned kPieces = (kRT + kCT) * kF16Tile * (kF16Step / 8);
+  constexpr int kPer = (kPieces + kThreads - 1) / kThreads;
+  __shared__ __align__(16) unsigned char lds[kF16Buffers][(kRT + kCT) * kF16TileBytes];
+  const unsigned lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  // Row blocks of a column block run side by side on one XCD (blockIdx % 8
+  // selects it), so that its L2 serves their common weights.
+  const unsigned nwg = gridDim.x, x = blockIdx.x % 8;
+  const unsigned v = x * (nwg / 8) + min(x, nwg % 8) + blockIdx.x / 8;
+  const unsigned row0 = (v % rowBlocks) * (kF16Tile * kRT);
+  const unsigned col0 = (v / rowBlocks) * (kF16Tile * kCT);
+  const unsigned steps = (p.inputWidth + kF16Step - 1) / kF16Step;
+
+  if (wave >= kRT * kCT) { // a loader
+    const unsigned tid = threadIdx.x - 64 * kRT * kCT;
+    const uint16_t *src[kPer];
+    unsigned at[kPer];
+    const unsigned piece = tid % 16; // of the row's step
+#pragma unroll
+    for (int e = 0; e < kPer; ++e) {
+      // staged row: the rows, then the columns (a piece past the last one
+      // repeats it)
+      const unsigned r = min((tid + e * kThreads) / 16, (kRT + kCT) * kF16Tile - 1);
+      src[e] = r < kRT * kF16Tile
+                   ? in + (size_t)min(row0 + r, p.tokens - 1) * p.inputWidth
+                   : w + (size_t)min(col0 + r - kRT * kF16Tile, p.rowCount - 1) * p.inputWidth;
+      at[e] = (r / kF16Tile) * kF16TileBytes + (piece / 4) * kF16ChunkBytes +
+              (r % kF16Tile) * 16 + (piece % 4) * 4;
+    }
+    uint4_t reg[kDepth][kPer];
+    auto load = [&](int slot, unsigned step) {
+      const unsigned k = step * kF16Step + 8 * piece;
+#pragma unroll
+      for (int e = 0; e < kPer; ++e)
+        reg[slot][e] = load_halves8<kVec>(src[e], k, p.inputWidth);
+    };
+    auto stage = [&](int slot, unsigned step) {
+      const bool past = step * kF16Step + 8 * piece >= p.inputWidth;
+      const unsigned buf = step % kF16Buffers;
+#pragma unroll
+      for (int e = 0; e < kPer; ++e) {
+        uint4_t d = reg[slot][e];
+        if (past)
+          d = uint4_t{0, 0, 0, 0};
+        unsigned char *to = lds[buf] + at[e];
+        *reinterpret_cast<uint32_t *>(to) = __builtin_amdgcn_perm(d[2], d[0], 0x05040100u);
+        *reinterpret_cast<uint32_t *>(to + 256) = __builtin_amdgcn_perm(d[2], d[0], 0x07060302u);
+        *reinterpret_cast<uint32_t *>(to + 512) = __builtin_amdgcn_perm(d[3], d[1], 0x05040100u);
+        *reinterpret_cast<uint32_t *>(to + 768) = __builtin_amdgcn_perm(d[3], d[1], 0x07060302u);
+      }
+    };
+    // Steps 0 and 1 staged ahead; inside the loop step s + 2, loads kDepth
+    // steps ahead of their staging.
+#pragma unroll
+    for (int d = 0; d < kDepth; ++d)
+      load(d, d); // (zeros past the end)
+    stage(0, 0);
+    load(0, kDepth);
+    stage(1 % kDepth, 1);
+    load(1 % kDepth, kDepth + 1);
+    lds_sync();
+    for (unsigned s0 = 0; s0 < steps; s0 += kDepth) {
+#pragma unroll
+      for (int d = 0; d < kDepth; ++d) {
+        const unsigned step = s0 + d;
+        if (step >= steps)
+          break;
+        if (step + 2 < steps) {
+          stage((d + 2) % kDepth, step + 2);
+          load((d + 2) % kDepth, step + 2 + kDepth);
+        }
+        lds_sync();
+      }
+    }
+    return;
+  }
+
+  const unsigned wr = wave / kCT, wc = wave % kCT; // the wave's tile
+  const bool live = row0 + wr * kF16Tile < p.tokens && col0 + wc * kF16Tile < p.rowCount;
+  v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  uint4_t qa[2], qb[2];
+  auto fetch = [&](int to, unsigned buf, unsigned c) {
+    const unsigned char *base = lds[buf] + lane * 16 + c * kF16ChunkBytes;
+    qa[to] = *reinterpret_cast<const uint4_t *>(base + wr * kF16TileBytes);
+    qb[to] = *reinterpret_cast<const uint4_t *>(base + (kRT + wc) * kF16TileBytes);
+  };
+  lds_sync();
+  fetch(0, 0, 0);
+  for (unsigned step = 0; step < steps; ++step) {
+    if (live) {
+#pragma unroll
+      for (unsigned c = 0; c < kF16Chunks; ++c) {
+        // The next chunk: the next step's first one was staged before the
+        // last barrier (after the last step it is read and not used).
+        if (c + 1 < kF16Chunks)
+          fetch((c + 1) % 2, step % kF16Buffers, c + 1);
+        else
+          fetch((c + 1) % 2, (step + 1) % kF16Buffers, 0);
+        // All conversions, then all products: alternating them costs 25 ns
+        // a product against 17.
+        float fa[8], fb[8];
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+          fa[s] = h2f((uint16_t)(qa[c % 2][s / 2] >> (16 * (s % 2))));
+          fb[s] = h2f((uint16_t)(qb[c % 2][s / 2] >> (16 * (s % 2))));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[s], fb[s], acc, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    asm volatile("s_barrier" ::: "memory");
+  }
+  if (!live)
+    return;
+  const unsigned g = lane / kF16Tile, col = col0 + kF16Tile * wc + lane % kF16Tile;
   if (col >= p.rowCount)
     return;
   const unsigned column = p.firstRow + col;
-  for (unsigned r = 0; r < nr; ++r)
-    store_linear(out, aux, bias, (size_t)(row0 + r) * p.outputWidth + column, column, p.epilogue,
-                 p.epilogueBlock, acc[r]);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const unsigned row = row0 + kF16Tile * wr + 4 * g + r;
+    if (row < p.tokens)
+      store_linear(out, aux, bias, (size_t)row * p.outputWidth + column, column, p.epilogue,
+                   p.epilogueBlock, acc[r]);
+  }
+}
+
+template <int kRT, int kCT, int kLoaders, int kDepth>
+void launch_linear_f16_as(const uint16_t *in, const uint16_t *w, void *out, const void *aux,
+                          const float *bias, const LinearParams &p, hipStream_t stream) {
+  const unsigned rowBlocks = (p.tokens + kF16Tile * kRT - 1) / (kF16Tile * kRT);
+  const unsigned colBlocks = (p.rowCount + kF16Tile * kCT - 1) / (kF16Tile * kCT);
+  const dim3 grid(rowBlocks * colBlocks), block(64 * (kRT * kCT + kLoaders));
+  if (p.inputWidth % 8 == 0 && aligned16(in) && aligned16(w))
+    hipLaunchKernelGGL((linear_f16_kernel<kRT, kCT, kLoaders, kDepth, true>), grid, block, 0,
+                       stream, in, w, out, aux, bias, p, rowBlocks);
+  else
+    hipLaunchKernelGGL((linear_f16_kernel<kRT, kCT, kLoaders, kDepth, false>), grid, block, 0,
+                       stream, in, w, out, aux, bias, p, rowBlocks);
 }
 
 } // namespace
@@ -181,9 +307,21 @@ hipError_t launch_copy_half_view(const uint16_t *src, uint16_t *out, const HalfV
 
 hipError_t launch_linear_f16(const uint16_t *in, const uint16_t *w, void *out, const void *aux,
                              const float *bias, const LinearParams &p, hipStream_t stream) {
-  const dim3 grid((p.rowCount + kF16Cols - 1) / kF16Cols, (p.tokens + kF16Rows - 1) / kF16Rows);
-  hipLaunchKernelGGL(linear_f16_kernel, grid, dim3(kF16Cols), 0, stream, in, w, out, aux, bias,
-                     p);
+  // Up to kF16FewTiles 16 x 16 tiles a tile a workgroup spreads the chains
+  // (8192 columns of 2560 for one row: 17.5 us against 21.9 with four column
+  // tiles a workgroup and 20.4 with 2 x 2; 2560 columns of 9216 for 33 rows:
+  // 55 against 72 and 65). Past that four waves share what a workgroup stages:
+  // four column tiles while there is one row of tiles (248,320 columns: 346 us
+  // against 366 and 404), else 2 x 2 (9216 columns of 2560, 93 rows: 62 us
+  // against 82 with 1 x 4 and 95 with one tile).
+  const unsigned rowTiles = (p.tokens + kF16Tile - 1) / kF16Tile;
+  const uint64_t tiles = (uint64_t)rowTiles * ((p.rowCount + kF16Tile - 1) / kF16Tile);
+  if (tiles <= kF16FewTiles)
+    launch_linear_f16_as<1, 1, 2, 4>(in, w, out, aux, bias, p, stream);
+  else if (rowTiles == 1)
+    launch_linear_f16_as<1, 4, 4, 4>(in, w, out, aux, bias, p, stream);
+  else
+    launch_linear_f16_as<2, 2, 4, 3>(in, w, out, aux, bias, p, stream);
   return hipGetLastError();
 }
 

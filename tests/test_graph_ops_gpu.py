@@ -91,6 +91,26 @@ def test_linear_f16_bit_exact(gpu, tokens, k, columns):
     assert np.array_equal(_host_u16(out), oracle.linear_f16(x, w))
 
 
+# Each tile layout at its edges (16 x 16 tiles, 128-wide steps of 32-wide
+# chunks): a tile a workgroup up to 512 tiles, 1 x 4 tiles past that for up to
+# 16 rows, else 2 x 2; ragged rows, columns and k, rows that are not 16-byte
+# aligned. Magnitudes over 2^-12 .. 2^8, so that a sum in another order or
+# with another rounding differs.
+@pytest.mark.parametrize("tokens,k,columns", [
+    (16, 128, 8192), (16, 264, 8208), (3, 133, 8201), (33, 200, 2752), (31, 136, 4200),
+    (48, 8, 2736), (65, 641, 1700), (17, 392, 256)])
+def test_linear_f16_tilings_bit_exact(gpu, tokens, k, columns):
+    print(f"linearF16 tiling tokens={tokens} k={k} columns={columns}", flush=True)
+    r = np.random.default_rng(tokens + k + columns)
+    spread = lambda *shape: _f16(r.standard_normal(shape) * 2.0 ** r.integers(-12, 9, shape))
+    x, w = spread(tokens, k), _f16(r.standard_normal((columns, k)) * 2.0 **
+                                   r.integers(-12, 1, (columns, k)))
+    out = torch.full((tokens, columns), 7.0, dtype=torch.float16, device=gpu)
+    ops.linear_f16(_u16_dev(x, gpu), _u16_dev(w, gpu), out)
+    torch.cuda.synchronize()
+    assert np.array_equal(_host_u16(out), oracle.linear_f16(x, w))
+
+
 @pytest.mark.parametrize("epilogue", [1, 2, 3, 4, 5, 6])
 def test_linear_f16_epilogues_bit_exact(gpu, epilogue):
     r = np.random.default_rng(epilogue)
