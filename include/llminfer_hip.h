@@ -283,9 +283,13 @@ LLMI_HIP_API int llmi_hip_gated_rms_norm_activated(const uint16_t *input, const 
  *   out      [T][Hq][d] fp16
  *   O[t,h] = softmax_j(q[t,h] . k[j,h/(Hq/Hkv)] / sqrt(d)) v[j,...], j <= P+t
  * Softmax and accumulation are fp32; the output is rounded to fp16 once.
- * `workspace` must hold llmi_hip_gqa_workspace_bytes(p) bytes (0 = none
- * needed): the split-K decode's per-split partials, written and read
- * within the call, so its contents between calls do not matter. */
+ * `workspace` holds llmi_hip_gqa_workspace_bytes(p) bytes (0 = none
+ * needed): the per-split partials of the split-K decode, or of a prefill
+ * whose keys are divided over more workgroups than its rows fill (a short
+ * chunk on a long history), written and read within the call, so its
+ * contents between calls do not matter. The decode (T == 1) needs it; a
+ * prefill without it (or with one that is smaller or not 16-byte aligned)
+ * runs undivided, which sums in another order. */
 LLMI_HIP_API int llmi_hip_causal_gqa(const uint16_t *q, const uint16_t *k_cache,
                         const uint16_t *v_cache, uint16_t *out, GqaParams p,
                         void *workspace, size_t workspace_bytes, void *stream);
@@ -314,7 +318,8 @@ LLMI_HIP_API int llmi_hip_kv_append_causal_gqa(const uint16_t *q, const uint16_t
  * partials go to a static device array of LLMI_HIP_NOALLOC_SCRATCH_BYTES
  * that each device the library runs on holds until the process ends; a
  * shape whose partials need more returns LLMI_HIP_WORKSPACE before any
- * launch (the north-star shapes need at most 2.1 MB). Calls that overlap on
+ * launch (the north-star shapes need at most 2.1 MB). T > 1 runs the append
+ * and the undivided prefill, without the array. Calls that overlap on
  * one device share that array and race; calls on one stream are ordered. */
 #define LLMI_HIP_NOALLOC_SCRATCH_BYTES (8u << 20)
 LLMI_HIP_API int llmi_hip_kv_append_causal_gqa_noalloc(const uint16_t *q,
@@ -342,7 +347,10 @@ LLMI_HIP_API int llmi_hip_kv_append_causal_gqa_noalloc(const uint16_t *q,
  * run in that order. T == 1 is one decode launch (plus its merge) that does
  * all of it; T > 1 normRopes K into the cache and appends V (two launches),
  * then runs the MFMA prefill with the q normRope in its query load and the
- * gate in its output store. Workspace: llmi_hip_gqa_workspace_bytes(p).
+ * gate in its output store, or, where the prefill divides its keys, normRope
+ * of q into the workspace, the prefill and its gating merge. Workspace:
+ * llmi_hip_gqa_workspace_bytes(p), as for llmi_hip_causal_gqa (the bits are
+ * those of that call with as large a workspace).
  * Supported: d 128 or 256, Hq/Hkv 2 or 4 (decode) or <= 4 (prefill),
  * rotary_dim a multiple of 16 up to d; other shapes return UNSUPPORTED. */
 LLMI_HIP_API int llmi_hip_gated_attention(const uint16_t *q_proj, const uint16_t *k_proj,

@@ -628,12 +628,22 @@ size_t llmi_hip_gqa_workspace_bytes(GqaParams p) {
   if (select_gqa(p) == GqaKernel::Decode)
     return decode_workspace_bytes(
         {p.tokens, p.queryHeads, p.kvHeads, p.headDim, p.past});
+  if (select_gqa(p) == GqaKernel::Prefill)
+    return prefill_workspace_bytes(
+        {p.tokens, p.queryHeads, p.kvHeads, p.headDim, p.past});
   return 0;
 }
 
 } // extern "C"
 
 namespace llmi {
+
+// Whether a prefill divides its keys: its shape calls for it and the caller
+// brought the workspace (callers without one get the undivided kernels).
+static bool run_prefill_split(const GqaShape &s, const void *workspace, size_t bytes) {
+  return workspace && aligned16(workspace) && prefill_split(s) &&
+         bytes >= prefill_workspace_bytes(s);
+}
 
 // CausalGqa with an optional fused KvAppend (k_new/v_new non-null).
 int run_gqa(const uint16_t *q, const uint16_t *k_new, const uint16_t *v_new,
@@ -671,6 +681,9 @@ int run_gqa(const uint16_t *q, const uint16_t *k_new, const uint16_t *v_new,
     if (r != LLMI_HIP_OK)
       return r;
   }
+  if (kind == GqaKernel::Prefill && run_prefill_split(s, workspace, workspace_bytes))
+    return launched(launch_gqa_prefill_split(q, k_cache, v_cache, out, workspace, s, nullptr, st),
+                    "gqaPrefillMfma");
   if (kind == GqaKernel::Prefill)
     return launched(launch_gqa_prefill(q, k_cache, v_cache, out, s, st),
                     "gqaPrefillMfma");
@@ -750,7 +763,18 @@ static int gated_attention(const uint16_t *q_proj, const uint16_t *k_proj,
     if (r == LLMI_HIP_OK)
       r = launched(launch_cache_append(v_new, v_cache, p.tokens * row, p.past * row, st),
                    "cacheAppend");
-    if (r == LLMI_HIP_OK)
+    if (r == LLMI_HIP_OK && run_prefill_split(s, workspace, workspace_bytes)) {
+      // The normalised query rows go through the workspace (each would
+      // otherwise be formed once a split); the merge gates.
+      uint16_t *rows = reinterpret_cast<uint16_t *>(static_cast<char *>(workspace) +
+                                                    prefill_split_partial_bytes(s));
+      RopeShape qs = rope_shape(p.tokens * p.queryHeads, p.queryHeads, p.headDim, rotary_dim,
+                                2 * p.headDim, p.past, 0, epsilon, theta, true);
+      r = launched(launch_norm_rope(q_proj, q_weight, rows, qs, st), "normRope");
+      if (r == LLMI_HIP_OK)
+        r = launched(launch_gqa_prefill_split(rows, k_cache, v_cache, out, workspace, s, &ga, st),
+                     "gqaPrefillGated");
+    } else if (r == LLMI_HIP_OK)
       r = launched(launch_gqa_prefill_gated(k_cache, v_cache, out, s, ga, st),
                    "gqaPrefillGated");
     return r;
@@ -974,7 +998,7 @@ unsigned llmi_hip_dispatch_count(int op, const void *params) {
       return 0;
     if (select_gqa(p) == GqaKernel::Decode)
       return decode_launches({p.tokens, p.queryHeads, p.kvHeads, p.headDim, p.past});
-    return 1;
+    return 1; // (the merge of a prefill that divides its keys belongs to it)
   }
   case LLMI_HIP_OP_KV_APPEND_CAUSAL_GQA: {
     const GqaParams &p = *static_cast<const GqaParams *>(params);

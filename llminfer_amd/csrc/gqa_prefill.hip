@@ -36,10 +36,15 @@
 // cycles per 32x32x16 MFMA with a 1 KB operand read each, against 38 with a
 // second wave on the SIMD and the reads two MFMAs ahead). The key-split
 // kernel gives each head a wave pair that splits the keys, at 248 registers.
+//
+// A grid that leaves CUs idle on a long history divides the keys over several
+// workgroups (SPLIT, split_plan): each leaves its partials in the caller's
+// workspace and gqa_prefill_merge_kernel combines and gates them.
 #include "hip_common.hpp"
 #include "kernels.hpp"
 #include "rope_gate.hpp"
 
+#include <algorithm>
 #include <math.h>
 #include <stdlib.h>
 #include <type_traits>
@@ -86,11 +91,12 @@ __device__ __forceinline__ half4_t read_tr(const char *base, unsigned off) {
 // for the few that miss the margin test, one per pass of the wave (as the
 // standalone gate kernel does). activated: the gate values are already
 // fp16(logistic(.)), and the output is their plain product (multiplyF16).
-__device__ __forceinline__ void gate_tile(half4_t (&v)[4], const half_t *g4p, bool activated) {
-  float g[16], sg[16];
+template <int N = 4>
+__device__ __forceinline__ void gate_tile(half4_t (&v)[N], const half_t *g4p, bool activated) {
+  float g[4 * N], sg[4 * N];
   unsigned need = 0;
 #pragma unroll
-  for (int g4 = 0; g4 < 4; ++g4) {
+  for (int g4 = 0; g4 < N; ++g4) {
     const half4_t gv = *reinterpret_cast<const half4_t *>(g4p + 8 * g4);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -104,15 +110,15 @@ __device__ __forceinline__ void gate_tile(half4_t (&v)[4], const half_t *g4p, bo
     need &= need - 1;
     float gk = g[0];
 #pragma unroll
-    for (int e = 1; e < 16; ++e)
+    for (int e = 1; e < 4 * N; ++e)
       gk = k == (unsigned)e ? g[e] : gk;
     const float sk = logistic_exact(gk);
 #pragma unroll
-    for (int e = 0; e < 16; ++e)
+    for (int e = 0; e < 4 * N; ++e)
       sg[e] = k == (unsigned)e ? sk : sg[e];
   }
 #pragma unroll
-  for (int g4 = 0; g4 < 4; ++g4)
+  for (int g4 = 0; g4 < N; ++g4)
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       v[g4][e] = __builtin_bit_cast(half_t, f2h(mul32(round16(sg[4 * g4 + e]), (float)v[g4][e])));
@@ -120,19 +126,52 @@ __device__ __forceinline__ void gate_tile(half4_t (&v)[4], const half_t *g4p, bo
 
 struct NoRows {}; // the ungated kernel's (empty) row argument
 
+// A split launch's partials: for each (split, token block, query head) the
+// block's 32 row references m and denominators l, and the unnormalised
+// O^T / (2^m) tile as the kernels hold it ([output tile][register][lane]).
+struct SplitArgs {
+  float *ml, *o;
+  unsigned splits;
+};
+// A split launch's workgroups in order of their keys: those that read the
+// same ones (a KV head's split: its head groups and row blocks) run side by
+// side on one XCD (blockIdx % 8 selects it), whose L2 then serves all but the
+// first (61 tokens on 16411 past rows, cold: 34.7 -> 30.2 us against a KV
+// head's head pairs on XCDs of their own).
+struct SplitPlace {
+  unsigned split, kvh, heads, rows;
+};
+__device__ __forceinline__ SplitPlace split_place(unsigned Hkv, unsigned groups, unsigned blocks) {
+  const unsigned nwg = gridDim.x, x = blockIdx.x % 8, members = groups * blocks;
+  const unsigned v = x * (nwg / 8) + min(x, nwg % 8) + blockIdx.x / 8;
+  const unsigned m = v % members, g = v / members;
+  return {g / Hkv, g % Hkv, m % groups, m / groups};
+}
+
+__device__ __forceinline__ size_t split_unit(unsigned split, unsigned nb, unsigned block,
+                                             unsigned Hq, unsigned h) {
+  return ((size_t)split * nb + block) * Hq + h;
+}
+
 // GATED: the query rows come from the projected q (per head D query values,
 // then D gate values) through normRope, staged in the K/V buffers before
 // the keys need them, and the output goes through the sigmoid gate: the
 // bits of the standalone normRope and sigmoidMul (rope_gate.hpp) around the
 // same attention.
-template <int D, int HW, bool GATED>
+// SPLIT: the block's tiles are divided over sa.splits workgroups, each of
+// which leaves its (m, l, O^T) for gqa_prefill_merge_kernel. The host gives a
+// split at least three tiles, so that its first one is visible to every row
+// of the block (the mask reaches into the last two tiles at most).
+template <int D, int HW, bool GATED, bool SPLIT>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * HW, 64 * HW),
                           amdgpu_waves_per_eu(HW > 4 ? 2 : 1, HW > 4 ? 2 : 1)))
 void gqa_prefill_kernel(const half_t *__restrict__ q, const half_t *__restrict__ kc,
                         const half_t *__restrict__ vc, half_t *__restrict__ out,
                         unsigned T, unsigned Hq, unsigned Hkv, unsigned P,
                         unsigned groups, unsigned nb, float c,
-                        typename std::conditional<GATED, GatedRows, NoRows>::type ga) {
+                        typename std::conditional<GATED, GatedRows, NoRows>::type ga,
+                        typename std::conditional<SPLIT, SplitArgs, NoRows>::type sa) {
+  static_assert(!(GATED && SPLIT), "the merge gates a split launch's rows");
   constexpr int KS = D / 16;         // k-steps of S^T over channels
   constexpr int DT = D / 32;         // 32-channel output tiles
   constexpr int ROWB = 2 * D;        // bytes per K/V row
@@ -157,8 +196,11 @@ void gqa_prefill_kernel(const half_t *__restrict__ q, const half_t *__restrict__
   // holds their K/V; token blocks go longest (most keys) first.
   const unsigned NH = Hkv * groups;
   const unsigned id = blockIdx.x, xcd = id % 8, j8 = id / 8;
-  unsigned hg, tbr;
-  if (8 % NH == 0 && nb % (8 / NH) == 0) {
+  unsigned hg, tbr, split = 0;
+  if constexpr (SPLIT) {
+    const SplitPlace at = split_place(Hkv, groups, nb);
+    hg = at.kvh * groups + at.heads, tbr = at.rows, split = at.split;
+  } else if (8 % NH == 0 && nb % (8 / NH) == 0) {
     const unsigned X = 8 / NH;
     hg = xcd / X;
     tbr = j8 * X + xcd % X;
@@ -178,8 +220,13 @@ void gqa_prefill_kernel(const half_t *__restrict__ q, const half_t *__restrict__
   const unsigned t0 = tb * BM, tq = t0 + r;
   const bool rowValid = tq < T;
   const unsigned tLast = min(t0 + BM, T) - 1;
-  const unsigned kend = P + tLast + 1; // keys [0, kend) can be visible
-  const unsigned tiles = (kend + BN - 1) / BN;
+  unsigned kend = P + tLast + 1; // keys [0, kend) can be visible
+  unsigned tbeg = 0, tiles = (kend + BN - 1) / BN; // this workgroup's [tbeg, tiles)
+  if constexpr (SPLIT) {
+    tbeg = (unsigned)((uint64_t)tiles * split / sa.splits);
+    tiles = (unsigned)((uint64_t)tiles * (split + 1) / sa.splits);
+    kend = min(kend, tiles * BN);
+  }
   const size_t rowBytes = (size_t)Hkv * D * 2;
   const char *kbase = reinterpret_cast<const char *>(kc) + (size_t)kvh * D * 2;
   const char *vbase = reinterpret_cast<const char *>(vc) + (size_t)kvh * D * 2;
@@ -452,7 +499,7 @@ void gqa_prefill_kernel(const half_t *__restrict__ q, const half_t *__restrict__
     const float tm = fmaxf(pr.a, pr.b) * c;
     const bool need = tm - mRef > kRaise;
     const float mNew = need ? tm - kHeadroom : mRef;
-    const float alpha = fast_exp2(mRef - mNew);
+    const float alpha = SPLIT && !need ? 1.0f : fast_exp2(mRef - mNew);
     mRef = mNew;
     raised = __builtin_amdgcn_ballot_w64(need) != 0;
     return alpha;
@@ -474,7 +521,7 @@ void gqa_prefill_kernel(const half_t *__restrict__ q, const half_t *__restrict__
       return load8(reinterpret_cast<const half_t *>(sk + kread[st % 4] + 128 * (st / 4) +
                                                     32 * ROWB * kt));
     };
-    const float negm = -mRef;
+    const float negm = SPLIT && mRef == -INFINITY ? 0.0f : -mRef;
     constexpr int AHEAD = 3;
     half8_t ka[AHEAD + 1][2];
 #pragma unroll
@@ -543,23 +590,23 @@ void gqa_prefill_kernel(const half_t *__restrict__ q, const half_t *__restrict__
     }
   }
   __syncthreads();
-  issue_k(0, sK0);
+  issue_k(tbeg, sK0);
   if constexpr (kStagedV)
-    load_v(0);
+    load_v(tbeg);
   else
-    issue_v(0, sV0);
+    issue_v(tbeg, sV0);
   wait_loads();
   __syncthreads();
-  if (tiles > 1)
-    issue_k(1, sK1);
+  if (tiles > tbeg + 1)
+    issue_k(tbeg + 1, sK1);
 
-  // Tile 0: scores and reference only (O is still zero).
+  // The first tile: scores and reference only (O is still zero).
   float sv[32]; // scores of the last tile, raw (masked keys -inf)
   {
     float16_t init[2], sacc[2];
-    const bool masked = BN > P + t0 + 1;
+    const bool masked = (tbeg + 1) * BN > P + t0 + 1;
     if (masked)
-      mask_init(0, init);
+      mask_init(tbeg * BN, init);
     const float zero[32] = {};
     phase_a(sK0, masked ? init : nullptr, zero, sacc, [](int) {});
     float mx = -INFINITY;
@@ -607,8 +654,8 @@ void gqa_prefill_kernel(const half_t *__restrict__ q, const half_t *__restrict__
     }
   };
   // Tiles [1, iu) lie wholly below the block's first query.
-  const unsigned iu = max(1u, min(tiles, (P + t0 + 1) / BN));
-  unsigned i = 1;
+  const unsigned iu = max(tbeg + 1, min(tiles, (P + t0 + 1) / BN));
+  unsigned i = tbeg + 1;
   for (; i + 1 < iu; i += 2) {
     step(i, false, sK1, sV0, sK0, sV1);
     step(i + 1, false, sK0, sV1, sK1, sV0);
@@ -621,22 +668,36 @@ void gqa_prefill_kernel(const half_t *__restrict__ q, const half_t *__restrict__
       step(i + 1, true, sK0, sV1, sK1, sV0);
   }
   {
-    const float negm = -mRef;
+    const float negm = SPLIT && mRef == -INFINITY ? 0.0f : -mRef;
 #pragma unroll
     for (int j = 0; j < 32; ++j)
       prob(sv, j, negm);
   }
   wait_loads();
   if constexpr (kStagedV)
-    store_vt((tiles - 1) % 2 == 0 ? sV0 : sV1);
+    store_vt((tiles - 1 - tbeg) % 2 == 0 ? sV0 : sV1);
   __syncthreads();
-  if ((tiles - 1) % 2 == 0)
+  if ((tiles - 1 - tbeg) % 2 == 0)
     pv(sV0);
   else
     pv(sV1);
 
   if (!rowValid)
     return;
+  if constexpr (SPLIT) {
+    const size_t u = split_unit(split, nb, tb, Hq, h);
+    if (hi == 0) {
+      sa.ml[u * 2 * BM + r] = mRef;
+      sa.ml[u * 2 * BM + BM + r] = lacc[0];
+    }
+    float *o = sa.o + u * BM * D + lane;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        o[(dt * 16 + v) * 64] = oacc[dt][v];
+    return;
+  }
   const float inv = 1.0f / lacc[0];
   half_t *orow = out + ((size_t)tq * Hq + h) * D;
 #pragma unroll
@@ -675,13 +736,18 @@ void gqa_prefill_kernel(const half_t *__restrict__ q, const half_t *__restrict__
 // rows go through normRope in LDS before the loop (the workgroup's 512
 // threads share the rows, the scales and one cos/sin table per block), the
 // output through the sigmoid gate.
-template <bool GATED>
+// SPLIT as in gqa_prefill_kernel, over the pair's steps: a workgroup leaves
+// the (m, l, O^T) that its wave pairs merged (m = -inf, l = 0, O = 0 for rows
+// that see none of its keys).
+template <bool GATED, bool SPLIT>
 __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2)))
 void gqa_prefill_halves_kernel(const half_t *__restrict__ q, const half_t *__restrict__ kc,
                                const half_t *__restrict__ vc, half_t *__restrict__ out,
                                unsigned T, unsigned Hq, unsigned Hkv, unsigned P,
                                unsigned hpairs, unsigned nb, float c,
-                               typename std::conditional<GATED, GatedRows, NoRows>::type ga) {
+                               typename std::conditional<GATED, GatedRows, NoRows>::type ga,
+                               typename std::conditional<SPLIT, SplitArgs, NoRows>::type sa) {
+  static_assert(!(GATED && SPLIT), "the merge gates a split launch's rows");
   constexpr int D = 256, KS = D / 16, DT = D / 32;
   constexpr int BK = 32;           // keys per tile
   constexpr int ROWB = 2 * D;      // bytes per K/V row
@@ -701,8 +767,11 @@ void gqa_prefill_halves_kernel(const half_t *__restrict__ q, const half_t *__res
   // holds their K/V.
   const unsigned NH = Hkv * hpairs, npairs = (nb + 1) / 2;
   const unsigned id = blockIdx.x, xcd = id % 8, j8 = id / 8;
-  unsigned hg, pr;
-  if (8 % NH == 0 && npairs % (8 / NH) == 0) {
+  unsigned hg, pr, split = 0;
+  if constexpr (SPLIT) {
+    const SplitPlace at = split_place(Hkv, hpairs, npairs);
+    hg = at.kvh * hpairs + at.heads, pr = at.rows, split = at.split;
+  } else if (8 % NH == 0 && npairs % (8 / NH) == 0) {
     const unsigned X = 8 / NH;
     hg = xcd / X;
     pr = j8 * X + xcd % X;
@@ -726,8 +795,14 @@ void gqa_prefill_halves_kernel(const half_t *__restrict__ q, const half_t *__res
   const bool rowValid = tq < T && !idle;
   // Keys [0, kend) can be visible to the long block; this wave's block needs
   // its first `mine` tiles.
-  const unsigned kend = P + min(bL * BM + BM, T);
-  const unsigned ntiles = (kend + BK - 1) / BK, steps = (ntiles + 1) / 2;
+  unsigned kend = P + min(bL * BM + BM, T);
+  const unsigned ntiles = (kend + BK - 1) / BK;
+  unsigned sbeg = 0, steps = (ntiles + 1) / 2; // this workgroup's [sbeg, steps)
+  if constexpr (SPLIT) {
+    sbeg = (unsigned)((uint64_t)steps * split / sa.splits);
+    steps = (unsigned)((uint64_t)steps * (split + 1) / sa.splits);
+    kend = min(kend, steps * 2 * BK);
+  }
   const unsigned mine = idle ? 0u : (P + min(t0 + BM, T) + BK - 1) / BK;
   const unsigned ju = (P + t0 + 1) / BK; // tiles [0, ju) need no mask
   const size_t rowBytes = (size_t)Hkv * D * 2;
@@ -998,10 +1073,10 @@ void gqa_prefill_halves_kernel(const half_t *__restrict__ q, const half_t *__res
     }
   }
   __syncthreads();
-  load_tile(kbase, 0, koff, sK00);
-  load_tile(kbase, 1, koff, sK01);
-  load_tile(vbase, 0, voff, sV00);
-  load_tile(vbase, 1, voff, sV01);
+  load_tile(kbase, 2 * sbeg, koff, sK00);
+  load_tile(kbase, 2 * sbeg + 1, koff, sK01);
+  load_tile(vbase, 2 * sbeg, voff, sV00);
+  load_tile(vbase, 2 * sbeg + 1, voff, sV01);
 
   // Step s: set s % 2 holds K and V of tiles 2s and 2s + 1; the other set
   // receives those of 2s + 2 and 2s + 3, requested as the step begins. Each
@@ -1026,7 +1101,7 @@ void gqa_prefill_halves_kernel(const half_t *__restrict__ q, const half_t *__res
         pv(vc_);
       }
     };
-    unsigned s = 0;
+    unsigned s = sbeg;
     for (; s + 1 < steps; s += 2) {
       step(s, k0, v0, sK10, sK11, sV10, sV11);
       step(s + 1, k1, v1, sK00, sK01, sV00, sV01);
@@ -1059,9 +1134,27 @@ void gqa_prefill_halves_kernel(const half_t *__restrict__ q, const half_t *__res
   if (half == 1 || !rowValid)
     return;
   const float m1 = sML[pi][0][lane], l1 = sML[pi][1][lane];
-  const float M = fmaxf(mRef, m1); // mRef is finite: key 0 is visible to every row
-  const float a0 = fast_exp2(mRef - M), a1 = fast_exp2(m1 - M);
+  // (unsplit, mRef is finite: key 0 is visible to every row)
+  const float M = fmaxf(mRef, m1);
+  const bool none = SPLIT && M == -INFINITY;
+  const float a0 = none ? 0.0f : fast_exp2(mRef - M), a1 = none ? 0.0f : fast_exp2(m1 - M);
   const LanePair lp = pair32(lsum * a0 + l1 * a1);
+  if constexpr (SPLIT) {
+    const size_t u = split_unit(split, nb, blk ? bS : bL, Hq, h);
+    if (hi == 0) {
+      sa.ml[u * 2 * BM + r] = M;
+      sa.ml[u * 2 * BM + BM + r] = lp.a + lp.b;
+    }
+    float *o = sa.o + u * BM * D + lane;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      const float *o1 = reinterpret_cast<const float *>(dt < 4 ? ma : mb) + (dt % 4) * 16 * 64;
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        o[(dt * 16 + v) * 64] = oacc[dt][v] * a0 + o1[v * 64 + lane] * a1;
+    }
+    return;
+  }
   const float inv = 1.0f / (lp.a + lp.b);
   half_t *orow = out + ((size_t)tq * Hq + h) * D;
 #pragma unroll
@@ -1084,35 +1177,84 @@ void gqa_prefill_halves_kernel(const half_t *__restrict__ q, const half_t *__res
   }
 }
 
+// The merge of a split launch: a wave per (token block, query head, 32-channel
+// output tile, 8-channel half pair g4): lane (r, hi) owns row r and channels
+// 32 dt + 8 g4 + 4 hi + [0, 4). Every split's partials are rescaled to the
+// largest reference, as the kernels rescale their own; the gate follows.
+template <int D, bool GATED>
+__global__ __launch_bounds__(256) void gqa_prefill_merge_kernel(
+    const float *__restrict__ ml, const float *__restrict__ po, half_t *__restrict__ out,
+    unsigned T, unsigned Hq, unsigned nb, unsigned splits, const half_t *qproj,
+    unsigned activated) {
+  constexpr unsigned DT = D / 32;
+  const unsigned w = blockIdx.x * 4 + threadIdx.x / 64, lane = threadIdx.x % 64;
+  const unsigned g4 = w % 4, dt = (w / 4) % DT, bh = w / (4 * DT);
+  const unsigned h = bh % Hq, blk = bh / Hq, r = lane % 32, hi = lane / 32;
+  const unsigned tq = blk * BM + r;
+  if (blk >= nb || tq >= T)
+    return;
+  const size_t stride = (size_t)nb * Hq; // units a split
+  const float *m = ml + split_unit(0, nb, blk, Hq, h) * 2 * BM + r;
+  const float *o = po + split_unit(0, nb, blk, Hq, h) * BM * D + (dt * 16 + 4 * g4) * 64 + lane;
+  float M = -INFINITY;
+#pragma unroll 8
+  for (unsigned s = 0; s < splits; ++s)
+    M = fmaxf(M, m[s * stride * 2 * BM]);
+  float l = 0.0f, acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 8
+  for (unsigned s = 0; s < splits; ++s) {
+    const float a = fast_exp2(m[s * stride * 2 * BM] - M);
+    l = fmaf(m[s * stride * 2 * BM + BM], a, l);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      acc[e] = fmaf(o[s * stride * BM * D + e * 64], a, acc[e]);
+  }
+  const float inv = 1.0f / l;
+  half4_t v[1] = {half4_t{f16_of(acc[0] * inv), f16_of(acc[1] * inv), f16_of(acc[2] * inv),
+                          f16_of(acc[3] * inv)}};
+  const size_t ch = 32 * dt + 8 * g4 + 4 * hi;
+  if constexpr (GATED)
+    gate_tile<1>(v, qproj + ((size_t)tq * Hq + h) * 2 * D + D + ch, activated);
+  *reinterpret_cast<half4_t *>(out + ((size_t)tq * Hq + h) * D + ch) = v[0];
+}
+
 template <int D> constexpr unsigned heads_per_wg(unsigned G) {
   return G < (D == 256 ? 4u : 8u) ? G : (D == 256 ? 4u : 8u);
 }
 
-template <int D, int HW, bool GATED = false, typename Rows = NoRows>
+template <int D, int HW, bool GATED = false, bool SPLIT = false, typename Rows = NoRows>
 hipError_t launch_dw(const GqaShape &s, const uint16_t *q, const uint16_t *k,
                      const uint16_t *v, uint16_t *out, hipStream_t stream,
-                     const Rows &rows = Rows{}) {
+                     const Rows &rows = Rows{}, const SplitArgs &split = SplitArgs{}) {
   const float c = kLog2e / sqrtf((float)D);
   const unsigned G = s.Hq / s.Hkv, groups = G / HW, nb = (s.T + BM - 1) / BM;
-  hipLaunchKernelGGL((gqa_prefill_kernel<D, HW, GATED>), dim3(nb * s.Hkv * groups),
-                     dim3(64 * HW), 0, stream, reinterpret_cast<const half_t *>(q),
+  typename std::conditional<SPLIT, SplitArgs, NoRows>::type sa;
+  if constexpr (SPLIT)
+    sa = split;
+  hipLaunchKernelGGL((gqa_prefill_kernel<D, HW, GATED, SPLIT>),
+                     dim3(nb * s.Hkv * groups * (SPLIT ? split.splits : 1)), dim3(64 * HW), 0,
+                     stream, reinterpret_cast<const half_t *>(q),
                      reinterpret_cast<const half_t *>(k), reinterpret_cast<const half_t *>(v),
                      reinterpret_cast<half_t *>(out), s.T, s.Hq, s.Hkv, s.P, groups, nb, c,
-                     rows);
+                     rows, sa);
   return hipGetLastError();
 }
 
-template <bool GATED, typename Rows>
+template <bool GATED, bool SPLIT = false, typename Rows = NoRows>
 hipError_t launch_halves(const GqaShape &s, const uint16_t *q, const uint16_t *k,
                          const uint16_t *v, uint16_t *out, hipStream_t stream,
-                         const Rows &rows) {
+                         const Rows &rows = Rows{}, const SplitArgs &split = SplitArgs{}) {
   const float c = kLog2e / sqrtf(256.0f);
   const unsigned G = s.Hq / s.Hkv, hpairs = G / 2, nb = (s.T + BM - 1) / BM;
-  hipLaunchKernelGGL((gqa_prefill_halves_kernel<GATED>), dim3((nb + 1) / 2 * s.Hkv * hpairs),
-                     dim3(512), 0, stream, reinterpret_cast<const half_t *>(q),
+  typename std::conditional<SPLIT, SplitArgs, NoRows>::type sa;
+  if constexpr (SPLIT)
+    sa = split;
+  hipLaunchKernelGGL((gqa_prefill_halves_kernel<GATED, SPLIT>),
+                     dim3((nb + 1) / 2 * s.Hkv * hpairs * (SPLIT ? split.splits : 1)), dim3(512),
+                     0, stream, reinterpret_cast<const half_t *>(q),
                      reinterpret_cast<const half_t *>(k), reinterpret_cast<const half_t *>(v),
                      reinterpret_cast<half_t *>(out), s.T, s.Hq, s.Hkv, s.P, hpairs, nb, c,
-                     rows);
+                     rows, sa);
   return hipGetLastError();
 }
 
@@ -1170,13 +1312,90 @@ hipError_t launch_d(const GqaShape &s, const uint16_t *q, const uint16_t *k,
     return launch_dw<D, 2>(s, q, k, v, out, stream);
   case 4:
     if (D == 256 && use_halves(s))
-      return launch_halves<false>(s, q, k, v, out, stream, NoRows{});
+      return launch_halves<false>(s, q, k, v, out, stream);
     return launch_dw<D, 4>(s, q, k, v, out, stream);
   case 8:
     if constexpr (D == 128)
       return launch_dw<D, 8>(s, q, k, v, out, stream);
   }
   return hipErrorInvalidValue;
+}
+
+// The split of a prefill's keys. Without one a short chunk on a long history
+// keeps a few CUs busy (61 tokens, 16 / 4 heads: 8 workgroups, 391 us at
+// 16411 past rows at head_dim 256 and 290 at 128; split 37 and 26), so the
+// keys are divided until every CU has a workgroup. A split takes at least
+// kSplitSteps tiles of 64 keys, counted over the past rows, which every row
+// sees: its O^T is written out and merged for what it saves (2 tokens on 1024
+// rows: 32.8 us unsplit, 19.7 / 21.6 / 27.0 at 3 / 4 / 6 tiles a split; 512
+// tokens on 500: 31.7 unsplit, 33.8 at 3), so at 511 past rows and fewer
+// nothing is split. At head_dim 256 two blocks of rows and more run as the
+// key-split kernel's pairs.
+constexpr unsigned kSplitSteps = 4, kSplitWorkgroups = 256;
+static_assert(kSplitSteps >= 3, "a split's first tile is visible to every row of its block");
+
+struct SplitPlan {
+  unsigned splits = 1;
+  bool halves = false;
+};
+SplitPlan split_plan(const GqaShape &s) {
+  SplitPlan p;
+  if (s.T < 2 || !prefill_supported(s))
+    return p;
+  const unsigned G = s.Hq / s.Hkv, nb = (s.T + BM - 1) / BM;
+  const unsigned hw = s.D == 256 ? heads_per_wg<256>(G) : heads_per_wg<128>(G);
+  p.halves = s.D == 256 && hw == 4 && nb >= 2;
+  const uint64_t base = p.halves ? (uint64_t)(nb + 1) / 2 * s.Hkv * (G / 2)
+                                 : (uint64_t)nb * s.Hkv * (G / hw);
+  const unsigned most = s.P / BN / kSplitSteps;
+  if (2 * base <= kSplitWorkgroups && most >= 2)
+    p.splits = std::min((unsigned)(kSplitWorkgroups / base), most);
+  return p;
+}
+
+template <int D>
+hipError_t launch_split_d(const GqaShape &s, const uint16_t *q, const uint16_t *k,
+                          const uint16_t *v, uint16_t *out, void *workspace,
+                          const GatedRows *ga, hipStream_t stream) {
+  const SplitPlan p = split_plan(s);
+  const unsigned nb = (s.T + BM - 1) / BM;
+  const size_t units = (size_t)p.splits * nb * s.Hq;
+  SplitArgs sa;
+  sa.ml = static_cast<float *>(workspace);
+  sa.o = sa.ml + units * 2 * BM;
+  sa.splits = p.splits;
+  hipError_t rc = hipErrorInvalidValue;
+  if (p.halves) {
+    rc = launch_halves<false, true>(s, q, k, v, out, stream, NoRows{}, sa);
+  } else {
+    switch (heads_per_wg<D>(s.Hq / s.Hkv)) {
+    case 1:
+      rc = launch_dw<D, 1, false, true>(s, q, k, v, out, stream, NoRows{}, sa);
+      break;
+    case 2:
+      rc = launch_dw<D, 2, false, true>(s, q, k, v, out, stream, NoRows{}, sa);
+      break;
+    case 4:
+      rc = launch_dw<D, 4, false, true>(s, q, k, v, out, stream, NoRows{}, sa);
+      break;
+    case 8:
+      if constexpr (D == 128)
+        rc = launch_dw<D, 8, false, true>(s, q, k, v, out, stream, NoRows{}, sa);
+      break;
+    }
+  }
+  if (rc != hipSuccess)
+    return rc;
+  const dim3 grid(nb * s.Hq * (D / 32)); // four waves a workgroup
+  half_t *o = reinterpret_cast<half_t *>(out);
+  if (ga)
+    hipLaunchKernelGGL((gqa_prefill_merge_kernel<D, true>), grid, dim3(256), 0, stream, sa.ml,
+                       sa.o, o, s.T, s.Hq, nb, p.splits,
+                       reinterpret_cast<const half_t *>(ga->qproj), ga->activated);
+  else
+    hipLaunchKernelGGL((gqa_prefill_merge_kernel<D, false>), grid, dim3(256), 0, stream, sa.ml,
+                       sa.o, o, s.T, s.Hq, nb, p.splits, (const half_t *)nullptr, 0u);
+  return hipGetLastError();
 }
 
 } // namespace
@@ -1216,6 +1435,27 @@ hipError_t launch_gqa_prefill(const uint16_t *q, const uint16_t *k,
   if (s.D == 128)
     return launch_d<128>(s, q, k, v, out, stream);
   return launch_d<256>(s, q, k, v, out, stream);
+}
+
+bool prefill_split(const GqaShape &s) { return split_plan(s).splits > 1; }
+
+// The partials, then (for the gated call) the normalised query rows.
+size_t prefill_split_partial_bytes(const GqaShape &s) {
+  const SplitPlan p = split_plan(s);
+  const size_t units = (size_t)p.splits * ((s.T + BM - 1) / BM) * s.Hq;
+  return p.splits > 1 ? units * BM * (2 + s.D) * sizeof(float) : 0;
+}
+size_t prefill_workspace_bytes(const GqaShape &s) {
+  const size_t partial = prefill_split_partial_bytes(s);
+  return partial ? partial + (size_t)s.T * s.Hq * s.D * 2 : 0;
+}
+
+hipError_t launch_gqa_prefill_split(const uint16_t *q, const uint16_t *k, const uint16_t *v,
+                                    uint16_t *out, void *workspace, const GqaShape &s,
+                                    const GatedRows *ga, hipStream_t stream) {
+  if (s.D == 128)
+    return launch_split_d<128>(s, q, k, v, out, workspace, ga, stream);
+  return launch_split_d<256>(s, q, k, v, out, workspace, ga, stream);
 }
 
 } // namespace llmi

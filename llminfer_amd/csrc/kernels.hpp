@@ -77,6 +77,16 @@ hipError_t launch_gqa_prefill_gated(const uint16_t *k, const uint16_t *v, uint16
 hipError_t launch_gqa_prefill(const uint16_t *q, const uint16_t *k,
                               const uint16_t *v, uint16_t *out,
                               const GqaShape &s, hipStream_t stream);
+// A prefill whose grid would leave CUs idle divides its keys over several
+// workgroups a block of rows, with a merge launch after it; it runs where the
+// caller's workspace holds prefill_workspace_bytes. ga: q are the normalised
+// rows (normRope's output) and the merge applies the gate of ga's rows.
+bool prefill_split(const GqaShape &s);
+size_t prefill_split_partial_bytes(const GqaShape &s); // the normalised rows lie behind
+size_t prefill_workspace_bytes(const GqaShape &s);
+hipError_t launch_gqa_prefill_split(const uint16_t *q, const uint16_t *k, const uint16_t *v,
+                                    uint16_t *out, void *workspace, const GqaShape &s,
+                                    const GatedRows *ga, hipStream_t stream);
 
 // Generic fallback for any head_dim <= 512 and any GQA ratio.
 bool generic_supported(const GqaShape &s);

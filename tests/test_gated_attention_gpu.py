@@ -85,6 +85,20 @@ def test_fused_block_equals_the_unfused_ops(gpu, T, past, shape, rot):
         assert names == ["normRopeTile", "cacheAppend", "gqaPrefillGated"]
 
 
+@pytest.mark.parametrize("T,past,shape,rot", [
+    (3, 515, (16, 4, 256), 64), (61, 1500, (16, 4, 256), 128), (40, 700, (16, 4, 128), 32)])
+def test_divided_block_equals_the_unfused_ops(gpu, T, past, shape, rot):
+    """A prefill that divides its keys: q normalised into the workspace, the
+    merge gates."""
+    hq, hkv, d = shape
+    print(f"divided gated attention T={T} past={past} shape={shape} rot={rot}", flush=True)
+    x, q_proj, k_proj, qw, kw = _case(600 + T + past, T, hq, hkv, d, past)
+    ref, out, caches_ref, caches = _run_both(gpu, x, q_proj, k_proj, qw, kw, past, rot)
+    assert torch.equal(caches_ref[0], caches[0]) and torch.equal(caches_ref[1], caches[1])
+    assert torch.equal(ref, out), "output differs from the unfused ops"
+    assert _lib.load().llmi_hip_gqa_workspace_bytes(_lib.GqaParams(T, hq, hkv, d, past)) > 0
+
+
 @pytest.mark.parametrize("T,past,hq,hkv", [(1, 4096, 16, 4), (40, 24, 16, 4), (100, 37, 64, 16)])
 def test_fused_block_against_the_oracle(gpu, T, past, hq, hkv):
     d, rot = 256, 64

@@ -182,6 +182,37 @@ def test_prefill_cfg3_every_token(gpu):
     print(f"  max abs err over {T} tokens x 16 heads: {err:.3g}", flush=True)
 
 
+# The keys divided over workgroups: from 512 past rows, one block of rows (the
+# single-wave kernel, any head_dim and group) or pairs of blocks (the key-split
+# kernel: even, odd and ragged counts), few splits and many, a ragged last tile.
+@pytest.mark.parametrize("shape,T,past", [
+    ((16, 4, 256), 2, 512), ((16, 4, 256), 32, 1031), ((16, 4, 256), 33, 777),
+    ((16, 4, 256), 70, 1024), ((16, 4, 256), 97, 2000), ((16, 4, 256), 5, 8200),
+    ((4, 2, 256), 20, 900), ((16, 4, 128), 45, 1111), ((8, 1, 128), 40, 703),
+    ((8, 8, 128), 33, 600)])
+def test_prefill_divided_keys(gpu, shape, T, past):
+    hq, hkv, d = shape
+    print(f"prefill divided shape={shape} T={T} past={past}", flush=True)
+    lib = _lib.load()
+    x = oracle.make_gqa_inputs(400 + T + past, T, hq, hkv, d, past)
+    # scores that grow along the keys, so that the splits' references differ
+    pos = np.arange(past + T, dtype=np.float32)[:, None, None]
+    x.k_cache = oracle.f32_to_f16(oracle.f16_to_f32(x.k_cache) * (0.5 + pos / (past + T)))
+    p = _lib.GqaParams(T, hq, hkv, d, past)
+    need = lib.llmi_hip_gqa_workspace_bytes(p)
+    assert need > 0, "not divided"
+    q, kc, vc = (u16_to_torch(a, gpu) for a in (x.q, x.k_cache, x.v_cache))
+    ws = torch.full((need,), 0xFF, dtype=torch.uint8, device=gpu)  # NaN patterns
+    want = oracle.gqa_dense_f64(x.q, x.k_cache, x.v_cache, past)
+    for size in (need, need - 1, 0):  # divided; undivided without enough workspace
+        out = torch.empty_like(q)
+        _lib.check(lib.llmi_hip_causal_gqa(q.data_ptr(), kc.data_ptr(), vc.data_ptr(),
+                                           out.data_ptr(), p, ws.data_ptr() if size else None,
+                                           size, torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        _check(oracle.f16_to_f32(torch_to_u16(out)).astype(np.float64), want)
+
+
 @pytest.mark.parametrize("growth,qscale", [(2.0, 1.0), (0.0, 4.0), (6.0, 2.0)])
 def test_prefill_moving_reference(gpu, growth, qscale):
     """Scores that keep growing along the keys (key rows scaled up with their
