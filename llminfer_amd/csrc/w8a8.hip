@@ -18,10 +18,9 @@
 //    meet by the xor butterfly, which is the reference's arithmetic order, so
 //    outputs are its bits. Eight groups' weight loads go out before their
 //    arithmetic.
-//  * GEMM (several rows): the reference's 8 lanes per column. Below 16 rows,
-//    a lane holds 4 rows and a weight group is loaded once for them; from 16
-//    rows the group dots come from int8 MFMA over 32 x 32 tiles, with the 8
-//    lanes' fp32 sums kept apart and merged in the butterfly's order.
+//  * GEMM (several rows): the group dots come from int8 MFMA over 32 x 32
+//    tiles, with the reference's 8 lanes' fp32 sums kept apart and merged in
+//    the butterfly's order.
 #include "exact_fp.hpp"
 #include "gated_norm.hpp"
 #include "hip_common.hpp"
@@ -426,74 +425,37 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemv_split_kernel(
 
 // ------------------------------------------------------------------- GEMM
 
-constexpr int kGemmLanes = 8, kGemmCols = 256 / kGemmLanes, kGemmRows = 4;
-
-__global__ __launch_bounds__(256) void gemm_kernel(
-    const int8_t *__restrict__ act, const float *__restrict__ as, const int8_t *__restrict__ w,
-    const uint16_t *__restrict__ ws, void *out, const void *aux, const float *bias, W8Args p) {
-  const unsigned col = blockIdx.x * kGemmCols + threadIdx.x / kGemmLanes;
-  const unsigned l = threadIdx.x % kGemmLanes;
-  const unsigned row0 = blockIdx.y * kGemmRows;
-  const unsigned nr = min((unsigned)kGemmRows, p.rows - row0);
-  float acc[kGemmRows] = {0.0f, 0.0f, 0.0f, 0.0f};
-  if (col < p.columns) {
-    const uint4_t *wrow = reinterpret_cast<const uint4_t *>(w + (size_t)col * p.groups * kGroup);
-    const uint16_t *wsrow = ws + (size_t)col * p.groups;
-    for (unsigned g = l; g < p.groups; g += kGemmLanes) {
-      const uint4_t w0 = __builtin_nontemporal_load(wrow + 2 * g);
-      const uint4_t w1 = __builtin_nontemporal_load(wrow + 2 * g + 1);
-      const float wsv = h2f(wsrow[g]);
-#pragma unroll
-      for (int r = 0; r < kGemmRows; ++r) {
-        const unsigned row = row0 + min((unsigned)r, nr - 1); // clamped: in bounds
-        const uint4_t *arow =
-            reinterpret_cast<const uint4_t *>(act + ((size_t)row * p.groups + g) * kGroup);
-        const int dot = group_dot(arow[0], arow[1], w0, w1);
-        if ((unsigned)r < nr)
-          acc[r] = add_term(acc[r], dot, as[(size_t)row * p.groups + g], wsv);
-      }
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < kGemmRows; ++r)
-#pragma unroll
-    for (int m = kGemmLanes / 2; m >= 1; m /= 2)
-      acc[r] = __fadd_rn(acc[r], __shfl_xor(acc[r], m, kGemmLanes));
-  if (l == 0 && col < p.columns) {
-    const unsigned column = p.firstRow + col;
-    for (unsigned r = 0; r < nr; ++r)
-      store_linear(out, aux, bias, (size_t)(row0 + r) * p.outputWidth + column, column,
-                   p.epilogue, p.block, acc[r]);
-  }
-}
-
-// ------------------------------------------------------------- MFMA GEMM
-
-// Many rows (prefill): the group dots come from v_mfma_i32_32x32x32_i8, one
-// instruction per 32-row x 32-column tile and group (K = 32 is exactly one
-// group, so each int32 result is the group's exact dot), and the VALU adds
-// (float(dot) * a) * w to fp32 sums. The reference's GEMM gives each output 8
-// lanes, lane l summing groups l, l + 8, ... in order before the xor
-// butterfly; here those 8 lane classes are split over the workgroup's waves
-// (wave w takes the groups g = w (mod waves), i.e. classes w and w + 4 with 4
-// waves, class w with 8), each class keeping its own fp32 sum per output, and
-// the sums meet through LDS in the butterfly's order
-// ((c0 + c4) + (c2 + c6)) + ((c1 + c5) + (c3 + c7)). So the bits are the
-// reference's. The per-element fp32 work (convert, two products, add: 4 VALU
-// operations per output and group) is the floor of the kernel.
+// Several rows (prefill, a short message): the group dots come from
+// v_mfma_i32_32x32x32_i8, one instruction per 32-row x 32-column tile and
+// group (K = 32 is exactly one group, so each int32 result is the group's
+// exact dot), and the VALU adds (float(dot) * a) * w to fp32 sums. The
+// reference's GEMM gives each output 8 lanes, lane l summing groups l, l + 8,
+// ... in order before the xor butterfly; here those 8 lane classes are a
+// workgroup's eight waves (wave w the groups g = w mod 8), and the sums meet
+// through LDS in the butterfly's order ((c0 + c4) + (c2 + c6)) + ((c1 + c5) +
+// (c3 + c7)). So the bits are the reference's.
 //
-// Staging: a step covers kPer groups per wave, i.e. (waves x kPer x 32)
-// consecutive bytes of each of the tile's 32 activation rows and 32 weight
-// rows, plus their scales. Each thread loads 16-byte chunks of each operand
-// (whole cache lines per row) kDepth - 1 steps ahead into registers and
-// writes them to the other of two LDS buffers, before the current step's
-// arithmetic (kEarly) or after it; one barrier a step. Rows are padded by 16
-// bytes so the MFMA operand reads (lane i: row i % 32) meet no bank
-// conflicts. Large grids (at least kMfmaManyTiles tiles) take 8 waves, one
-// group each a step, loads one step ahead, staged early: 71 VGPRs, so three
-// workgroups share a CU. Small grids (the 2560-column down projection) take
-// loads three steps ahead, staged late, which hides more latency inside a
-// workgroup when few workgroups share a CU.
+// Bounds: from a few hundred rows the fp32 work that this order demands, per
+// output and group a conversion (2.3 ns a wave64 operation a SIMD), two
+// products (1.2 each) and an addition (1.5): 36 us for 512 rows of a 2560 ->
+// 9216 projection, where the kernel takes 60; below that the latency of a
+// step. So waves in flight decide: a tile a workgroup, 64 registers and 37 KB
+// of LDS, four workgroups a CU.
+//
+// A step covers 8 groups: 256 bytes of each of the tile's 32 activation and 32
+// weight rows go HBM -> LDS with buffer loads that write LDS directly, double
+// buffered; the scales come through registers, requested a step before they
+// are staged. One barrier a step, and no wait there for the scales.
+// Measured (weights rotating past the MALL; 512 rows of 2560 -> 9216, 512 of
+// 9216 -> 2560, 128 of 2560 -> 9216, 13 of 9216 -> 2560):
+//   through registers and a padded layout      74.4, 73.4, 24.5, 58.1 us
+//   this                                       60.5, 61.1, 19.5, 21.2 us
+// (the fourth ran a kernel of four rows a lane). Not kept: 64 x 32, 32 x 64
+// and 64 x 64 tiles (61 - 65 us at 512 rows with half the loads, but four or
+// two waves a SIMD; 33 and 49 us at 13 rows); three and four buffers (64 - 90
+// us: fewer workgroups a CU); the row scales by DPP broadcast inside the
+// product (a DPP product takes 2.0 ns: 71 us); dots accumulated onto 1.5 x
+// 2^23 so that a subtraction stands for the conversion (16 registers more: 67).
 //
 // Operand layout: lane i supplies row (column) i % 32 of the tile and the
 // 16 bytes (i / 32) * 16 of the group for both operands; any K order shared
@@ -505,153 +467,140 @@ __global__ __launch_bounds__(256) void gemm_kernel(
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
-constexpr unsigned kTile = 32, kMfmaMinRows = 16, kMfmaManyTiles = 512;
+constexpr unsigned kTile = 32, kGemmThreads = 512;
+constexpr unsigned kSpan = 8, kStepBytes = kSpan * kGroup; // groups, bytes of a row a step
+constexpr unsigned kScalePitch = kTile + 4;                // staged scales a group
+constexpr int kBufferWord3 = 0x00020000;                   // gfx9 raw buffer descriptor, dword 3
 
-// A step stages kWaves * kPer groups; loads run kDepth - 1 steps ahead.
-template <int kWaves, int kPer, int kDepth> struct MfmaCfg {
-  static constexpr unsigned kSpan = kWaves * kPer;             // groups per step
-  static constexpr unsigned kPitch = kSpan * kGroup + 16;      // bytes per staged row
-  static constexpr unsigned kOperand = kTile * kPitch;         // one operand tile
-  static constexpr unsigned kScales = kSpan * kTile * 4;       // [group][32] fp32
-  static constexpr unsigned kBuffer = 2 * kOperand + 2 * kScales;
-  static constexpr unsigned kSums = kWaves * kTile * kTile * 4;
-  static constexpr unsigned kBytes = 2 * kBuffer > kSums ? 2 * kBuffer : kSums;
-};
+typedef __attribute__((address_space(3))) void lds_void_t;
 
-template <int kWaves, int kPer, int kDepth, bool kEarly>
-__global__ __launch_bounds__(64 * kWaves) void gemm_mfma_kernel(
+// Direct memory -> LDS load of 16 bytes per lane at base + offset (in bounds
+// up to `bytes`): lane i's bytes land at dst + 16 i (dst is wave-uniform).
+__device__ __forceinline__ void load_lds16(const void *base, unsigned bytes, unsigned char *dst,
+                                           unsigned offset) {
+  const __amdgpu_buffer_rsrc_t rsrc =
+      __builtin_amdgcn_make_buffer_rsrc((void *)base, (short)0, (int)bytes, kBufferWord3);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_t *)dst, 16, offset, 0, 0, 0);
+}
+
+__global__ __launch_bounds__(kGemmThreads, 4) void gemm_kernel(
     const int8_t *__restrict__ act, const float *__restrict__ as, const int8_t *__restrict__ w,
     const uint16_t *__restrict__ ws, void *out, const void *aux, const float *bias, W8Args p,
     unsigned rowTiles) {
-  using L = MfmaCfg<kWaves, kPer, kDepth>;
-  constexpr int kClasses = 8 / kWaves; // lane classes per wave
-  static_assert(L::kSpan % 8 == 0, "a step must hold whole sets of the 8 lane classes");
-  __shared__ __align__(16) unsigned char lds[L::kBytes];
-  const unsigned nwg = gridDim.x, b = blockIdx.x, x = b % 8;
-  const unsigned v = x * (nwg / 8) + min(x, nwg % 8) + b / 8;
+  // Two buffers (the activation rows, then the weight rows), named one by one
+  // so that the compiler can tell the loads in flight from the LDS reads.
+  __shared__ __align__(1024) unsigned char s0[2 * kTile * kStepBytes], s1[2 * kTile * kStepBytes];
+  __shared__ __align__(16) float sc[2][2 * kSpan * kScalePitch];
+  const unsigned nwg = gridDim.x, x = blockIdx.x % 8;
+  const unsigned v = x * (nwg / 8) + min(x, nwg % 8) + blockIdx.x / 8;
   const unsigned row0 = (v % rowTiles) * kTile, col0 = (v / rowTiles) * kTile;
-  const unsigned tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
-  const size_t k = (size_t)p.groups * kGroup;
-  const unsigned nsteps = (p.groups + L::kSpan - 1) / L::kSpan;
+  const unsigned tid = threadIdx.x, lane = tid % 64;
+  const unsigned wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const unsigned k = p.groups * kGroup;
+  const unsigned nsteps = (p.groups + kSpan - 1) / kSpan;
 
-  // Staging roles: chunks schunk + 2 * kWaves * j (16 bytes each, j < kPer)
-  // of one row of each operand; kPer scales of one row (column) for the
-  // first 32 * kWaves threads.
-  const unsigned srow = tid / (2 * kWaves), schunk = tid % (2 * kWaves);
-  const int8_t *sact = act + min(row0 + srow, p.rows - 1) * k + 16 * (schunk % 2);
-  const int8_t *swt = w + min(col0 + srow, p.columns - 1) * k + 16 * (schunk % 2);
-  const bool scaler = tid < kTile * kWaves;
-  const unsigned sr = tid / kWaves, sg = tid % kWaves;
-  const float *sas = as + (size_t)min(row0 + sr, p.rows - 1) * p.groups;
-  const uint16_t *sws = ws + (size_t)min(col0 + sr, p.columns - 1) * p.groups;
-  v4i ra[kDepth][kPer], rb[kDepth][kPer];
-  float rs[kDepth][kPer];
-  uint16_t rt[kDepth][kPer];
-  auto load = [&](int slot, unsigned step) {
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      const unsigned g = min(step * L::kSpan + schunk / 2 + kWaves * j, p.groups - 1); // clamped
-      ra[slot][j] = *reinterpret_cast<const v4i *>(sact + (size_t)g * kGroup);
-      rb[slot][j] = *reinterpret_cast<const v4i *>(swt + (size_t)g * kGroup);
-      if (scaler) {
-        const unsigned gs = min(step * L::kSpan + sg + kWaves * j, p.groups - 1);
-        rs[slot][j] = sas[gs];
-        rt[slot][j] = sws[gs];
-      }
-    }
+  // A wave moves four rows of each operand, a lane 16 bytes of one: slot s of
+  // row r holds chunk s ^ (r % 16), so the operand reads (32 rows, one chunk)
+  // meet no bank conflicts. Past a row's end the reads give the next row's
+  // bytes or, past the tensor's, nothing: groups that no wave uses.
+  const unsigned srow = 4 * wave + lane / 16, schunk = (lane % 16) ^ (srow % 16);
+  unsigned oa = min(row0 + srow, p.rows - 1) * k + 16 * schunk;
+  unsigned ob = min(col0 + srow, p.columns - 1) * k + 16 * schunk;
+  auto load = [&](unsigned char *to) { // the next step
+    load_lds16(act, p.rows * k, to + 4 * wave * kStepBytes, oa);
+    load_lds16(w, p.columns * k, to + (kTile + 4 * wave) * kStepBytes, ob);
+    oa += kStepBytes;
+    ob += kStepBytes;
   };
-  auto stage = [&](int slot, unsigned buf) {
-    unsigned char *base = lds + buf * L::kBuffer;
-    float *sc = reinterpret_cast<float *>(base + 2 * L::kOperand);
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      const unsigned at = srow * L::kPitch + 16 * (schunk + 2 * kWaves * j);
-      *reinterpret_cast<v4i *>(base + at) = ra[slot][j];
-      *reinterpret_cast<v4i *>(base + L::kOperand + at) = rb[slot][j];
-      if (scaler) {
-        sc[(sg + kWaves * j) * kTile + sr] = rs[slot][j];
-        sc[L::kSpan * kTile + (sg + kWaves * j) * kTile + sr] = h2f(rt[slot][j]);
-      }
-    }
+  // The first four waves an activation scale a thread, the others a weight's.
+  const bool act_scaler = wave < 4;
+  const unsigned sr = (tid % 256) / 8, sg = tid % 8;
+  const unsigned os = (act_scaler ? min(row0 + sr, p.rows - 1) : min(col0 + sr, p.columns - 1)) *
+                      p.groups;
+  uint32_t rs; // fp32 or fp16 bits as loaded
+  auto load_scale = [&](unsigned step) {
+    const unsigned g = min(step * kSpan + sg, p.groups - 1); // clamped past the end
+    if (act_scaler)
+      rs = reinterpret_cast<const uint32_t *>(as)[os + g];
+    else
+      rs = ws[os + g];
   };
-
-#pragma unroll
-  for (int d = 0; d < kDepth - 1; ++d)
-    if ((unsigned)d < nsteps)
-      load(d, d);
-  stage(0, 0);
-  __syncthreads();
+  auto stage_scale = [&](float *to) {
+    if (act_scaler)
+      to[sg * kScalePitch + sr] = __uint_as_float(rs);
+    else
+      to[(kSpan + sg) * kScalePitch + sr] = h2f((uint16_t)rs);
+  };
 
   const unsigned m = lane % kTile, h = lane / kTile;
+  const unsigned from = m * kStepBytes + 16 * ((2 * wave + h) ^ (m % 16));
   const v16i zero = {};
-  float acc[kClasses][16];
+  float acc[16];
 #pragma unroll
-  for (int c = 0; c < kClasses; ++c)
+  for (int r = 0; r < 16; ++r)
+    acc[r] = 0.0f;
+  // One step of this wave's group.
+  auto compute = [&](const unsigned char *st, const float *scl) {
+    const v4i a = *reinterpret_cast<const v4i *>(st + from);
+    const v4i b = *reinterpret_cast<const v4i *>(st + kTile * kStepBytes + from);
+    const v16i dots = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, zero, 0, 0, 0);
+    const float wsv = scl[(kSpan + wave) * kScalePitch + m];
+    const float4 *sa = reinterpret_cast<const float4 *>(scl + wave * kScalePitch + 4 * h);
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
-      acc[c][r] = 0.0f;
-  for (unsigned s0 = 0; s0 < nsteps; s0 += kDepth) {
-#pragma unroll
-    for (int d = 0; d < kDepth; ++d) {
-      const unsigned step = s0 + d;
-      if (step >= nsteps)
-        break;
-      if (step + kDepth - 1 < nsteps)
-        load((d + kDepth - 1) % kDepth, step + kDepth - 1);
-      // The other buffer was released by the previous step's barrier.
-      if (kEarly && step + 1 < nsteps)
-        stage((d + 1) % kDepth, (step + 1) % 2);
-      const unsigned char *base = lds + (step % 2) * L::kBuffer;
-      const float *sc = reinterpret_cast<const float *>(base + 2 * L::kOperand);
-#pragma unroll
-      for (int j = 0; j < kPer; ++j) {
-        const unsigned gl = wave + kWaves * j; // group within the step
-        if (step * L::kSpan + gl < p.groups) {
-          const unsigned off = m * L::kPitch + gl * kGroup + 16 * h;
-          const v4i a = *reinterpret_cast<const v4i *>(base + off);
-          const v4i bw = *reinterpret_cast<const v4i *>(base + L::kOperand + off);
-          const float wsv = sc[L::kSpan * kTile + gl * kTile + m];
-          const v16i dots = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, bw, zero, 0, 0, 0);
-          const float4 *sa = reinterpret_cast<const float4 *>(sc + gl * kTile + 4 * h);
-          const int c = j % kClasses;
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const float4 a4 = sa[2 * q];
-            acc[c][4 * q + 0] = add_term(acc[c][4 * q + 0], dots[4 * q + 0], a4.x, wsv);
-            acc[c][4 * q + 1] = add_term(acc[c][4 * q + 1], dots[4 * q + 1], a4.y, wsv);
-            acc[c][4 * q + 2] = add_term(acc[c][4 * q + 2], dots[4 * q + 2], a4.z, wsv);
-            acc[c][4 * q + 3] = add_term(acc[c][4 * q + 3], dots[4 * q + 3], a4.w, wsv);
-          }
-        }
-      }
-      if (!kEarly && step + 1 < nsteps)
-        stage((d + 1) % kDepth, (step + 1) % 2);
-      __syncthreads();
+    for (int q = 0; q < 4; ++q) {
+      const float4 a4 = sa[2 * q];
+      acc[4 * q + 0] = add_term(acc[4 * q + 0], dots[4 * q + 0], a4.x, wsv);
+      acc[4 * q + 1] = add_term(acc[4 * q + 1], dots[4 * q + 1], a4.y, wsv);
+      acc[4 * q + 2] = add_term(acc[4 * q + 2], dots[4 * q + 2], a4.z, wsv);
+      acc[4 * q + 3] = add_term(acc[4 * q + 3], dots[4 * q + 3], a4.w, wsv);
     }
+  };
+  // A step: the next one's loads go out, this one's arithmetic runs, the next
+  // one's scale (requested a step ago) is staged and the one after requested.
+  // The wait before the barrier is for everything but that last request.
+  auto run = [&](unsigned step, const unsigned char *st, unsigned char *next) {
+    if (step + 1 < nsteps)
+      load(next);
+    if (step * kSpan + wave < p.groups)
+      compute(st, sc[step % 2]);
+    stage_scale(sc[(step + 1) % 2]);
+    load_scale(step + 2);
+    asm volatile("s_waitcnt vmcnt(1) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+  load(s0);
+  load_scale(0);
+  stage_scale(sc[0]);
+  load_scale(1);
+  asm volatile("s_waitcnt vmcnt(1) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  for (unsigned step = 0; step < nsteps; step += 2) {
+    run(step, s0, s1);
+    if (step + 1 < nsteps)
+      run(step + 1, s1, s0);
   }
 
-  float *sums = reinterpret_cast<float *>(lds) + wave * kTile * kTile;
+  // The classes of half a tile (16 rows) at a time meet in LDS, in the
+  // butterfly's order.
+  float *sums = reinterpret_cast<float *>(s0);
+  constexpr unsigned T = kTile * kTile / 2;
+  static_assert(sizeof s0 >= kSpan * T * sizeof(float) && T == kGemmThreads, "half a tile");
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const unsigned rr = 8 * (r / 4) + 4 * h + r % 4;
-    sums[rr * kTile + m] = kClasses == 2 ? __fadd_rn(acc[0][r], acc[kClasses - 1][r]) : acc[0][r];
-  }
-  __syncthreads();
-  for (unsigned e = tid; e < kTile * kTile; e += 64 * kWaves) {
-    const unsigned row = row0 + e / kTile, col = col0 + e % kTile;
-    if (row >= p.rows || col >= p.columns)
-      continue;
-    const float *s = reinterpret_cast<const float *>(lds) + e;
-    constexpr unsigned T = kTile * kTile;
-    float total;
-    if (kWaves == 4) // wave w holds c_w + c_(w+4)
-      total = __fadd_rn(__fadd_rn(s[0], s[2 * T]), __fadd_rn(s[T], s[3 * T]));
-    else
-      total = __fadd_rn(__fadd_rn(__fadd_rn(s[0], s[4 * T]), __fadd_rn(s[2 * T], s[6 * T])),
-                        __fadd_rn(__fadd_rn(s[T], s[5 * T]), __fadd_rn(s[3 * T], s[7 * T])));
-    const unsigned column = p.firstRow + col;
-    store_linear(out, aux, bias, (size_t)row * p.outputWidth + column, column, p.epilogue,
-                 p.block, total);
+  for (int half = 0; half < 2; ++half) {
+    if (half)
+      lds_sync();
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+      sums[wave * T + (8 * (r / 4) + 4 * h + r % 4) * kTile + m] = acc[8 * half + r];
+    lds_sync();
+    const unsigned row = row0 + 16 * half + tid / kTile, col = col0 + tid % kTile;
+    if (row < p.rows && col < p.columns) {
+      const float *c = sums + tid;
+      const float total =
+          __fadd_rn(__fadd_rn(__fadd_rn(c[0], c[4 * T]), __fadd_rn(c[2 * T], c[6 * T])),
+                    __fadd_rn(__fadd_rn(c[T], c[5 * T]), __fadd_rn(c[3 * T], c[7 * T])));
+      const unsigned column = p.firstRow + col;
+      store_linear(out, aux, bias, (size_t)row * p.outputWidth + column, column, p.epilogue,
+                   p.block, total);
+    }
   }
 }
 
@@ -1069,20 +1018,11 @@ hipError_t launch_linear_w8a8(const int8_t *act, const float *as, const int8_t *
   else if (s.rows == 1)
     hipLaunchKernelGGL(gemv_kernel, dim3((s.columns + kGemvCols - 1) / kGemvCols),
                        dim3(kGemvThreads), 0, stream, act, as, w, ws, out, aux, bias, a);
-  else if (s.rows >= kMfmaMinRows) {
+  else {
     const unsigned rowTiles = (s.rows + kTile - 1) / kTile;
-    const unsigned tiles = rowTiles * ((s.columns + kTile - 1) / kTile);
-    if (tiles >= kMfmaManyTiles)
-      hipLaunchKernelGGL((gemm_mfma_kernel<8, 1, 2, true>), dim3(tiles), dim3(512), 0, stream,
-                         act, as, w, ws, out, aux, bias, a, rowTiles);
-    else
-      hipLaunchKernelGGL((gemm_mfma_kernel<8, 1, 4, false>), dim3(tiles), dim3(512), 0, stream,
-                         act, as, w, ws, out, aux, bias, a, rowTiles);
-  } else
-    hipLaunchKernelGGL(gemm_kernel,
-                       dim3((s.columns + kGemmCols - 1) / kGemmCols,
-                            (s.rows + kGemmRows - 1) / kGemmRows),
-                       dim3(256), 0, stream, act, as, w, ws, out, aux, bias, a);
+    hipLaunchKernelGGL(gemm_kernel, dim3(rowTiles * ((s.columns + kTile - 1) / kTile)),
+                       dim3(kGemmThreads), 0, stream, act, as, w, ws, out, aux, bias, a, rowTiles);
+  }
   return hipGetLastError();
 }
 
