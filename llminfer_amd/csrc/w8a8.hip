@@ -543,16 +543,19 @@ __global__ __launch_bounds__(kGemmThreads, 4) void gemm_kernel(
   auto compute = [&](const unsigned char *st, const float *scl) {
     const v4i a = *reinterpret_cast<const v4i *>(st + from);
     const v4i b = *reinterpret_cast<const v4i *>(st + kTile * kStepBytes + from);
-    const v16i dots = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, zero, 0, 0, 0);
     const float wsv = scl[(kSpan + wave) * kScalePitch + m];
+    const v16i dots = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, zero, 0, 0, 0);
     const float4 *sa = reinterpret_cast<const float4 *>(scl + wave * kScalePitch + 4 * h);
+    float4 a4[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      a4[q] = sa[2 * q];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const float4 a4 = sa[2 * q];
-      acc[4 * q + 0] = add_term(acc[4 * q + 0], dots[4 * q + 0], a4.x, wsv);
-      acc[4 * q + 1] = add_term(acc[4 * q + 1], dots[4 * q + 1], a4.y, wsv);
-      acc[4 * q + 2] = add_term(acc[4 * q + 2], dots[4 * q + 2], a4.z, wsv);
-      acc[4 * q + 3] = add_term(acc[4 * q + 3], dots[4 * q + 3], a4.w, wsv);
+      acc[4 * q + 0] = add_term(acc[4 * q + 0], dots[4 * q + 0], a4[q].x, wsv);
+      acc[4 * q + 1] = add_term(acc[4 * q + 1], dots[4 * q + 1], a4[q].y, wsv);
+      acc[4 * q + 2] = add_term(acc[4 * q + 2], dots[4 * q + 2], a4[q].z, wsv);
+      acc[4 * q + 3] = add_term(acc[4 * q + 3], dots[4 * q + 3], a4[q].w, wsv);
     }
   };
   // A step: the next one's loads go out, this one's arithmetic runs, the next
