@@ -345,10 +345,9 @@ LLMI_HIP_API int llmi_hip_kv_append_causal_gqa_noalloc(const uint16_t *q,
  * out, k_cache and v_cache are bit-identical to llmi_hip_norm_rope (q and
  * k), llmi_hip_cache_append, llmi_hip_causal_gqa and llmi_hip_sigmoid_mul
  * run in that order. T == 1 is one decode launch (plus its merge) that does
- * all of it; T > 1 normRopes K into the cache and appends V (two launches),
- * then runs the MFMA prefill with the q normRope in its query load and the
- * gate in its output store, or, where the prefill divides its keys, normRope
- * of q into the workspace, the prefill and its gating merge. Workspace:
+ * all of it; T > 1 normRopes q into out and K into the cache and appends V
+ * (one launch), then runs the MFMA prefill of out's rows with the gate in its
+ * output store, or in its merge where it divides its keys. Workspace:
  * llmi_hip_gqa_workspace_bytes(p), as for llmi_hip_causal_gqa (the bits are
  * those of that call with as large a workspace).
  * Supported: d 128 or 256, Hq/Hkv 2 or 4 (decode) or <= 4 (prefill),

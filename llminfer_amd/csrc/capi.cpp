@@ -682,7 +682,7 @@ int run_gqa(const uint16_t *q, const uint16_t *k_new, const uint16_t *v_new,
       return r;
   }
   if (kind == GqaKernel::Prefill && run_prefill_split(s, workspace, workspace_bytes))
-    return launched(launch_gqa_prefill_split(q, k_cache, v_cache, out, workspace, s, nullptr, st),
+    return launched(launch_gqa_prefill_split(q, k_cache, v_cache, out, workspace, s, nullptr, 0, st),
                     "gqaPrefillMfma");
   if (kind == GqaKernel::Prefill)
     return launched(launch_gqa_prefill(q, k_cache, v_cache, out, s, st),
@@ -759,23 +759,21 @@ static int gated_attention(const uint16_t *q_proj, const uint16_t *k_proj,
     const unsigned row = p.kvHeads * p.headDim;
     RopeShape ks = rope_shape(p.tokens * p.kvHeads, p.kvHeads, p.headDim, rotary_dim,
                               p.headDim, p.past, p.past * p.kvHeads, epsilon, theta, true);
-    int r = launched(launch_norm_rope(k_proj, k_weight, k_cache, ks, st), "normRope");
-    if (r == LLMI_HIP_OK)
-      r = launched(launch_cache_append(v_new, v_cache, p.tokens * row, p.past * row, st),
-                   "cacheAppend");
-    if (r == LLMI_HIP_OK && run_prefill_split(s, workspace, workspace_bytes)) {
-      // The normalised query rows go through the workspace (each would
-      // otherwise be formed once a split); the merge gates.
-      uint16_t *rows = reinterpret_cast<uint16_t *>(static_cast<char *>(workspace) +
-                                                    prefill_split_partial_bytes(s));
-      RopeShape qs = rope_shape(p.tokens * p.queryHeads, p.queryHeads, p.headDim, rotary_dim,
-                                2 * p.headDim, p.past, 0, epsilon, theta, true);
-      r = launched(launch_norm_rope(q_proj, q_weight, rows, qs, st), "normRope");
-      if (r == LLMI_HIP_OK)
-        r = launched(launch_gqa_prefill_split(rows, k_cache, v_cache, out, workspace, s, &ga, st),
-                     "gqaPrefillGated");
-    } else if (r == LLMI_HIP_OK)
-      r = launched(launch_gqa_prefill_gated(k_cache, v_cache, out, s, ga, st),
+    // The normalised query rows go through the output: each is read back only
+    // by the wave that then writes it, or before the merge writes any.
+    RopeShape qs = rope_shape(p.tokens * p.queryHeads, p.queryHeads, p.headDim, rotary_dim,
+                              2 * p.headDim, p.past, 0, epsilon, theta, true);
+    int r = launched(launch_attention_rows(q_proj, q_weight, out, qs, k_proj, k_weight, k_cache,
+                                           ks, v_new, v_cache + (size_t)p.past * row,
+                                           p.tokens * row, st),
+                     "normRope");
+    if (r == LLMI_HIP_OK && run_prefill_split(s, workspace, workspace_bytes))
+      r = launched(launch_gqa_prefill_split(out, k_cache, v_cache, out, workspace, s, q_proj,
+                                            ga.activated, st),
+                   "gqaPrefillGated");
+    else if (r == LLMI_HIP_OK)
+      r = launched(launch_gqa_prefill_gated(out, k_cache, v_cache, out, s, q_proj, ga.activated,
+                                            st),
                    "gqaPrefillGated");
     return r;
   }

@@ -40,6 +40,10 @@
 // A grid that leaves CUs idle on a long history divides the keys over several
 // workgroups (SPLIT, split_plan): each leaves its partials in the caller's
 // workspace and gqa_prefill_merge_kernel combines and gates them.
+//
+// The gated call's query rows are normalised by a launch of their own, into
+// the output (launch_attention_rows): inside these kernels, one or two waves a
+// SIMD, that work took 22 us (333 tokens: 47.5 us with it, 25.5 without).
 #include "hip_common.hpp"
 #include "kernels.hpp"
 #include "rope_gate.hpp"
@@ -124,7 +128,14 @@ __device__ __forceinline__ void gate_tile(half4_t (&v)[N], const half_t *g4p, bo
       v[g4][e] = __builtin_bit_cast(half_t, f2h(mul32(round16(sg[4 * g4 + e]), (float)v[g4][e])));
 }
 
-struct NoRows {}; // the ungated kernel's (empty) row argument
+struct NoArgs {}; // an argument the kernel's form does not take
+
+// GATED: the projected rows (per head D query values, then D gate values)
+// whose gates the output goes through.
+struct GateArgs {
+  const half_t *qproj;
+  unsigned activated;
+};
 
 // A split launch's partials: for each (split, token block, query head) the
 // block's 32 row references m and denominators l, and the unnormalised
@@ -153,11 +164,9 @@ __device__ __forceinline__ size_t split_unit(unsigned split, unsigned nb, unsign
   return ((size_t)split * nb + block) * Hq + h;
 }
 
-// GATED: the query rows come from the projected q (per head D query values,
-// then D gate values) through normRope, staged in the K/V buffers before
-// the keys need them, and the output goes through the sigmoid gate: the
-// bits of the standalone normRope and sigmoidMul (rope_gate.hpp) around the
-// same attention.
+// GATED: the output goes through the sigmoid gate, with the bits of the
+// standalone sigmoidMul. The query rows may be the output's own (the gated
+// call normalises them there): a wave reads the rows it writes, at its start.
 // SPLIT: the block's tiles are divided over sa.splits workgroups, each of
 // which leaves its (m, l, O^T) for gqa_prefill_merge_kernel. The host gives a
 // split at least three tiles, so that its first one is visible to every row
@@ -165,12 +174,12 @@ __device__ __forceinline__ size_t split_unit(unsigned split, unsigned nb, unsign
 template <int D, int HW, bool GATED, bool SPLIT>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * HW, 64 * HW),
                           amdgpu_waves_per_eu(HW > 4 ? 2 : 1, HW > 4 ? 2 : 1)))
-void gqa_prefill_kernel(const half_t *__restrict__ q, const half_t *__restrict__ kc,
-                        const half_t *__restrict__ vc, half_t *__restrict__ out,
+void gqa_prefill_kernel(const half_t *q, const half_t *__restrict__ kc,
+                        const half_t *__restrict__ vc, half_t *out,
                         unsigned T, unsigned Hq, unsigned Hkv, unsigned P,
                         unsigned groups, unsigned nb, float c,
-                        typename std::conditional<GATED, GatedRows, NoRows>::type ga,
-                        typename std::conditional<SPLIT, SplitArgs, NoRows>::type sa) {
+                        typename std::conditional<GATED, GateArgs, NoArgs>::type ga,
+                        typename std::conditional<SPLIT, SplitArgs, NoArgs>::type sa) {
   static_assert(!(GATED && SPLIT), "the merge gates a split launch's rows");
   constexpr int KS = D / 16;         // k-steps of S^T over channels
   constexpr int DT = D / 32;         // 32-channel output tiles
@@ -360,104 +369,10 @@ void gqa_prefill_kernel(const half_t *__restrict__ q, const half_t *__restrict__
   // Q^T as the MFMA B operand: lane holds query row r, channels
   // 16 s + 8 hi + [0, 8). Rows past T use zeros (their output is dropped).
   half8_t qb[KS];
-  if constexpr (GATED) {
-    // Each wave's 32 query rows through normRope in its own K/V buffer
-    // (rows of D + 8 halves, then their scales). The (1 + w) weights and the
-    // (token, pair) table of fp16 cos/sin, the same for every head of the
-    // block, are made once per workgroup after wave 0's rows. The buffers
-    // are cleared for the keys afterwards.
-    static_assert(HW <= 4, "one K/V buffer per wave");
-    constexpr unsigned PITCH = D + 8, CPR = D / 8;
-    char *buf = wave == 0 ? sK0 : wave == 1 ? sK1 : wave == 2 ? sV0 : sV1;
-    uint16_t *rows = reinterpret_cast<uint16_t *>(buf);
-    float *scl = reinterpret_cast<float *>(rows + BM * PITCH);
-    float *w1 = reinterpret_cast<float *>(sK0 + BM * PITCH * 2 + BM * 4);
-    half2_t *cs = reinterpret_cast<half2_t *>(w1 + D); // fp16 values, stored exactly
-    const unsigned half = ga.rot / 2, nrow = min((unsigned)BM, T - t0);
-    const half_t *qp = reinterpret_cast<const half_t *>(ga.qproj);
-    for (unsigned i = lane; i < nrow * CPR; i += 64) {
-      const unsigned rr = i / CPR, cc = i % CPR;
-      *reinterpret_cast<uint4_t *>(rows + rr * PITCH + 8 * cc) =
-          *reinterpret_cast<const uint4_t *>(qp + ((size_t)(t0 + rr) * Hq + h) * 2 * D + 8 * cc);
-    }
-    for (unsigned i = threadIdx.x; i < (unsigned)D; i += 64 * HW)
-      w1[i] = 1.0f + ga.qw[i];
-    for (unsigned e = threadIdx.x; e < nrow * half; e += 64 * HW) {
-      const unsigned tt = e / half, i = e % half;
-      const float2 v2 = rope_cos_sin(__fdiv_rn((float)(P + t0 + tt), ga.freqs[i]));
-      cs[e] = half2_t{(half_t)v2.x, (half_t)v2.y};
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if (lane < nrow) {
-      // The sequential chain; its row is read eight chunks ahead.
-      const uint4_t *row = reinterpret_cast<const uint4_t *>(rows + lane * PITCH);
-      float sum = 0.0f;
-      for (unsigned c8 = 0; c8 < CPR; c8 += 8) {
-        uint4_t x[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
-          x[u] = row[c8 + u];
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-          sum = sumsq8(x[u], sum);
-      }
-      scl[lane] = rms_scale_of(sum, D, ga.eps);
-    }
-    __syncthreads(); // the shared tables and every row's scale are in place
-    const unsigned pchunks = half / 8, rest = CPR - 2 * pchunks;
-    for (unsigned it = lane; it < nrow * pchunks; it += 64) {
-      const unsigned rr = it / pchunks, j0 = 8 * (it % pchunks), j1 = j0 + half;
-      uint16_t *row = rows + rr * PITCH;
-      const float scale = scl[rr];
-      const uint4_t qx = *reinterpret_cast<const uint4_t *>(row + j0);
-      const uint4_t qy = *reinterpret_cast<const uint4_t *>(row + j1);
-      uint4_t sx, sy;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const uint16_t bx = (uint16_t)(qx[e / 2] >> (16 * (e & 1)));
-        const uint16_t by = (uint16_t)(qy[e / 2] >> (16 * (e & 1)));
-        const float x = normed(bx, scale, w1[j0 + e]);
-        const float y = normed(by, scale, w1[j1 + e]);
-        const half2_t c2 = cs[rr * half + j0 + e];
-        const float2 t2 = make_float2((float)c2[0], (float)c2[1]);
-        const uint32_t ox = rotate_x(x, y, t2), oy = rotate_y(x, y, t2);
-        if (e & 1) {
-          sx[e / 2] |= ox << 16;
-          sy[e / 2] |= oy << 16;
-        } else {
-          sx[e / 2] = ox;
-          sy[e / 2] = oy;
-        }
-      }
-      *reinterpret_cast<uint4_t *>(row + j0) = sx;
-      *reinterpret_cast<uint4_t *>(row + j1) = sy;
-    }
-    for (unsigned it = lane; it < nrow * rest; it += 64) {
-      const unsigned rr = it / rest, j0 = 8 * (2 * pchunks + it % rest);
-      uint16_t *row = rows + rr * PITCH;
-      const float scale = scl[rr];
-      const uint4_t qx = *reinterpret_cast<const uint4_t *>(row + j0);
-      uint4_t sx;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint32_t lo = f2h(normed((uint16_t)(qx[e] & 0xFFFFu), scale, w1[j0 + 2 * e]));
-        const uint32_t hi = f2h(normed((uint16_t)(qx[e] >> 16), scale, w1[j0 + 2 * e + 1]));
-        sx[e] = lo | (hi << 16);
-      }
-      *reinterpret_cast<uint4_t *>(row + j0) = sx;
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
-      qb[s] = rowValid ? *reinterpret_cast<const half8_t *>(rows + r * PITCH + 16 * s + 8 * hi)
-                       : half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-    __syncthreads(); // every wave is done with its buffer before they are cleared
-  } else {
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
-      qb[s] = rowValid ? load8(q + ((size_t)tq * Hq + h) * D + 16 * s + 8 * hi)
-                       : half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-  }
+  for (int s = 0; s < KS; ++s)
+    qb[s] = rowValid ? load8(q + ((size_t)tq * Hq + h) * D + 16 * s + 8 * hi)
+                     : half8_t{0, 0, 0, 0, 0, 0, 0, 0};
 
   float16_t oacc[DT];
 #pragma unroll
@@ -708,7 +623,7 @@ void gqa_prefill_kernel(const half_t *__restrict__ q, const half_t *__restrict__
       v[g4] = half4_t{f16_of(oacc[dt][4 * g4 + 0] * inv), f16_of(oacc[dt][4 * g4 + 1] * inv),
                       f16_of(oacc[dt][4 * g4 + 2] * inv), f16_of(oacc[dt][4 * g4 + 3] * inv)};
     if constexpr (GATED)
-      gate_tile(v, reinterpret_cast<const half_t *>(ga.qproj) + ((size_t)tq * Hq + h) * 2 * D +
+      gate_tile(v, ga.qproj + ((size_t)tq * Hq + h) * 2 * D +
                        D + 32 * dt + 4 * hi, ga.activated);
 #pragma unroll
     for (int g4 = 0; g4 < 4; ++g4)
@@ -732,21 +647,18 @@ void gqa_prefill_kernel(const half_t *__restrict__ q, const half_t *__restrict__
 // multiply V (v_dot2). At the end each odd-tile wave hands its (m, l, O) to
 // its partner through LDS. One step = one barrier: the four tiles of the
 // next step (K and V of tiles 2s + 2 and 2s + 3, shared by both blocks) go
-// HBM -> LDS as the step begins. GATED as in gqa_prefill_kernel: the query
-// rows go through normRope in LDS before the loop (the workgroup's 512
-// threads share the rows, the scales and one cos/sin table per block), the
-// output through the sigmoid gate.
+// HBM -> LDS as the step begins. GATED as in gqa_prefill_kernel.
 // SPLIT as in gqa_prefill_kernel, over the pair's steps: a workgroup leaves
 // the (m, l, O^T) that its wave pairs merged (m = -inf, l = 0, O = 0 for rows
 // that see none of its keys).
 template <bool GATED, bool SPLIT>
 __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2)))
-void gqa_prefill_halves_kernel(const half_t *__restrict__ q, const half_t *__restrict__ kc,
-                               const half_t *__restrict__ vc, half_t *__restrict__ out,
+void gqa_prefill_halves_kernel(const half_t *q, const half_t *__restrict__ kc,
+                               const half_t *__restrict__ vc, half_t *out,
                                unsigned T, unsigned Hq, unsigned Hkv, unsigned P,
                                unsigned hpairs, unsigned nb, float c,
-                               typename std::conditional<GATED, GatedRows, NoRows>::type ga,
-                               typename std::conditional<SPLIT, SplitArgs, NoRows>::type sa) {
+                               typename std::conditional<GATED, GateArgs, NoArgs>::type ga,
+                               typename std::conditional<SPLIT, SplitArgs, NoArgs>::type sa) {
   static_assert(!(GATED && SPLIT), "the merge gates a split launch's rows");
   constexpr int D = 256, KS = D / 16, DT = D / 32;
   constexpr int BK = 32;           // keys per tile
@@ -759,8 +671,6 @@ void gqa_prefill_halves_kernel(const half_t *__restrict__ q, const half_t *__res
   __shared__ __attribute__((aligned(1024))) char sV00[TILEB], sV01[TILEB], sV10[TILEB],
       sV11[TILEB];
   __shared__ float sML[4][2][64];
-  // GATED: the (1 + w) weights, then the (token, pair) table of fp16 cos/sin.
-  __shared__ float sTab[GATED ? D + BM * (D / 2) : 1];
 
   // Workgroup -> (block pair, KV head, head pair): each XCD (workgroups are
   // dealt round-robin over 8) serves as few KV heads as possible, so its L2
@@ -845,128 +755,10 @@ void gqa_prefill_halves_kernel(const half_t *__restrict__ q, const half_t *__res
   opaque(vread[1]);
 
   half8_t qb[KS];
-  if constexpr (GATED) {
-    // (block, head) pair pp's row rr sits in buffer 2 pp + rr / 16 at
-    // (rr % 16) * PITCH (rows of D + 8 halves keep the per-row chains off
-    // one bank).
-    constexpr unsigned PITCH = D + 8, CPR = D / 8;
-    auto rowp = [&](unsigned pp, unsigned rr) {
-      const unsigned bsel = 2 * pp + rr / 16;
-      char *b = bsel == 0   ? sK00
-                : bsel == 1 ? sK01
-                : bsel == 2 ? sK10
-                : bsel == 3 ? sK11
-                : bsel == 4 ? sV00
-                : bsel == 5 ? sV01
-                : bsel == 6 ? sV10
-                            : sV11;
-      return reinterpret_cast<uint16_t *>(b) + (rr % 16) * PITCH;
-    };
-    const unsigned halfrot = ga.rot / 2;
-    const unsigned nrL = min((unsigned)BM, T - bL * BM), nrS = min((unsigned)BM, T - bS * BM);
-    auto nrow = [&](unsigned pp) { return pp < 2 ? nrL : nrS; };
-    auto first_tok = [&](unsigned pp) { return (pp < 2 ? bL : bS) * BM; };
-    const half_t *qp = reinterpret_cast<const half_t *>(ga.qproj);
-    for (unsigned i = threadIdx.x; i < 4 * BM * CPR; i += 512) {
-      const unsigned pp = i / (BM * CPR), rem = i % (BM * CPR);
-      const unsigned rr = rem / CPR, cc = rem % CPR;
-      if (rr < nrow(pp))
-        *reinterpret_cast<uint4_t *>(rowp(pp, rr) + 8 * cc) =
-            *reinterpret_cast<const uint4_t *>(
-                qp + ((size_t)(first_tok(pp) + rr) * Hq + (kvh * hpairs + hp) * 2 + pp % 2) *
-                         2 * D +
-                8 * cc);
-    }
-    float *w1 = sTab;
-    half2_t *cs = reinterpret_cast<half2_t *>(sTab + D); // fp16 values, stored exactly
-    for (unsigned i = threadIdx.x; i < (unsigned)D; i += 512)
-      w1[i] = 1.0f + ga.qw[i];
-    __syncthreads();
-    if (threadIdx.x < 4 * BM) {
-      // The sequential chain of one row; its chunks are read eight ahead.
-      const unsigned pp = threadIdx.x / BM, rr = threadIdx.x % BM;
-      if (rr < nrow(pp)) {
-        const uint4_t *row = reinterpret_cast<const uint4_t *>(rowp(pp, rr));
-        float sum = 0.0f;
-        for (unsigned c8 = 0; c8 < CPR; c8 += 8) {
-          uint4_t x[8];
 #pragma unroll
-          for (int u = 0; u < 8; ++u)
-            x[u] = row[c8 + u];
-#pragma unroll
-          for (int u = 0; u < 8; ++u)
-            sum = sumsq8(x[u], sum);
-        }
-        sML[pp][0][rr] = rms_scale_of(sum, D, ga.eps);
-      }
-    }
-    const unsigned pchunks = halfrot / 8, rest = CPR - 2 * pchunks;
-    for (unsigned bb = 0; bb < 2; ++bb) {
-      // The cos/sin table of this block's tokens, then its two heads' rows.
-      const unsigned tok0 = bb ? bS * BM : bL * BM, nr = bb ? nrS : nrL;
-      for (unsigned e = threadIdx.x; e < nr * halfrot; e += 512) {
-        const unsigned tt = e / halfrot, i = e % halfrot;
-        const float2 v2 = rope_cos_sin(__fdiv_rn((float)(P + tok0 + tt), ga.freqs[i]));
-        cs[e] = half2_t{(half_t)v2.x, (half_t)v2.y};
-      }
-      __syncthreads(); // the table (and, the first time, every scale)
-      for (unsigned it = threadIdx.x; it < 2 * nr * pchunks; it += 512) {
-        const unsigned pp = 2 * bb + it / (nr * pchunks), rem = it % (nr * pchunks);
-        const unsigned rr = rem / pchunks, j0 = 8 * (rem % pchunks), j1 = j0 + halfrot;
-        uint16_t *row = rowp(pp, rr);
-        const float scale = sML[pp][0][rr];
-        const uint4_t qx = *reinterpret_cast<const uint4_t *>(row + j0);
-        const uint4_t qy = *reinterpret_cast<const uint4_t *>(row + j1);
-        uint4_t sx, sy;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const uint16_t bx = (uint16_t)(qx[e / 2] >> (16 * (e & 1)));
-          const uint16_t by = (uint16_t)(qy[e / 2] >> (16 * (e & 1)));
-          const float x = normed(bx, scale, w1[j0 + e]);
-          const float y = normed(by, scale, w1[j1 + e]);
-          const half2_t c2 = cs[rr * halfrot + j0 + e];
-          const float2 t2 = make_float2((float)c2[0], (float)c2[1]);
-          const uint32_t ox = rotate_x(x, y, t2), oy = rotate_y(x, y, t2);
-          if (e & 1) {
-            sx[e / 2] |= ox << 16;
-            sy[e / 2] |= oy << 16;
-          } else {
-            sx[e / 2] = ox;
-            sy[e / 2] = oy;
-          }
-        }
-        *reinterpret_cast<uint4_t *>(row + j0) = sx;
-        *reinterpret_cast<uint4_t *>(row + j1) = sy;
-      }
-      for (unsigned it = threadIdx.x; it < 2 * nr * rest; it += 512) {
-        const unsigned pp = 2 * bb + it / (nr * rest), rem = it % (nr * rest);
-        const unsigned rr = rem / rest, j0 = 8 * (2 * pchunks + rem % rest);
-        uint16_t *row = rowp(pp, rr);
-        const float scale = sML[pp][0][rr];
-        const uint4_t qx = *reinterpret_cast<const uint4_t *>(row + j0);
-        uint4_t sx;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const uint32_t lo = f2h(normed((uint16_t)(qx[e] & 0xFFFFu), scale, w1[j0 + 2 * e]));
-          const uint32_t hi2 = f2h(normed((uint16_t)(qx[e] >> 16), scale, w1[j0 + 2 * e + 1]));
-          sx[e] = lo | (hi2 << 16);
-        }
-        *reinterpret_cast<uint4_t *>(row + j0) = sx;
-      }
-      __syncthreads(); // the table is free again
-    }
-    const uint16_t *myrow = rowp(pi, r);
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
-      qb[s] = rowValid ? *reinterpret_cast<const half8_t *>(myrow + 16 * s + 8 * hi)
-                       : half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-    __syncthreads(); // every wave has its rows before the buffers are cleared
-  } else {
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
-      qb[s] = rowValid ? load8(q + ((size_t)tq * Hq + h) * D + 16 * s + 8 * hi)
-                       : half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-  }
+  for (int s = 0; s < KS; ++s)
+    qb[s] = rowValid ? load8(q + ((size_t)tq * Hq + h) * D + 16 * s + 8 * hi)
+                     : half8_t{0, 0, 0, 0, 0, 0, 0, 0};
 
   float16_t oacc[DT];
 #pragma unroll
@@ -1169,7 +961,7 @@ void gqa_prefill_halves_kernel(const half_t *__restrict__ q, const half_t *__res
         v[g4][e] = f16_of((oacc[dt][i] * a0 + o1[i * 64 + lane] * a1) * inv);
       }
     if constexpr (GATED)
-      gate_tile(v, reinterpret_cast<const half_t *>(ga.qproj) + ((size_t)tq * Hq + h) * 2 * D +
+      gate_tile(v, ga.qproj + ((size_t)tq * Hq + h) * 2 * D +
                        D + 32 * dt + 4 * hi, ga.activated);
 #pragma unroll
     for (int g4 = 0; g4 < 4; ++g4)
@@ -1222,13 +1014,13 @@ template <int D> constexpr unsigned heads_per_wg(unsigned G) {
   return G < (D == 256 ? 4u : 8u) ? G : (D == 256 ? 4u : 8u);
 }
 
-template <int D, int HW, bool GATED = false, bool SPLIT = false, typename Rows = NoRows>
+template <int D, int HW, bool GATED = false, bool SPLIT = false, typename Rows = NoArgs>
 hipError_t launch_dw(const GqaShape &s, const uint16_t *q, const uint16_t *k,
                      const uint16_t *v, uint16_t *out, hipStream_t stream,
                      const Rows &rows = Rows{}, const SplitArgs &split = SplitArgs{}) {
   const float c = kLog2e / sqrtf((float)D);
   const unsigned G = s.Hq / s.Hkv, groups = G / HW, nb = (s.T + BM - 1) / BM;
-  typename std::conditional<SPLIT, SplitArgs, NoRows>::type sa;
+  typename std::conditional<SPLIT, SplitArgs, NoArgs>::type sa;
   if constexpr (SPLIT)
     sa = split;
   hipLaunchKernelGGL((gqa_prefill_kernel<D, HW, GATED, SPLIT>),
@@ -1240,13 +1032,13 @@ hipError_t launch_dw(const GqaShape &s, const uint16_t *q, const uint16_t *k,
   return hipGetLastError();
 }
 
-template <bool GATED, bool SPLIT = false, typename Rows = NoRows>
+template <bool GATED, bool SPLIT = false, typename Rows = NoArgs>
 hipError_t launch_halves(const GqaShape &s, const uint16_t *q, const uint16_t *k,
                          const uint16_t *v, uint16_t *out, hipStream_t stream,
                          const Rows &rows = Rows{}, const SplitArgs &split = SplitArgs{}) {
   const float c = kLog2e / sqrtf(256.0f);
   const unsigned G = s.Hq / s.Hkv, hpairs = G / 2, nb = (s.T + BM - 1) / BM;
-  typename std::conditional<SPLIT, SplitArgs, NoRows>::type sa;
+  typename std::conditional<SPLIT, SplitArgs, NoArgs>::type sa;
   if constexpr (SPLIT)
     sa = split;
   hipLaunchKernelGGL((gqa_prefill_halves_kernel<GATED, SPLIT>),
@@ -1287,17 +1079,18 @@ template <int D> unsigned prefill_heads(const GqaShape &s) {
 }
 
 template <int D>
-hipError_t launch_gated_d(const GqaShape &s, const uint16_t *k, const uint16_t *v,
-                          uint16_t *out, const GatedRows &ga, hipStream_t stream) {
+hipError_t launch_gated_d(const GqaShape &s, const uint16_t *q, const uint16_t *k,
+                          const uint16_t *v, uint16_t *out, const GateArgs &ga,
+                          hipStream_t stream) {
   switch (prefill_heads<D>(s)) {
   case 1:
-    return launch_dw<D, 1, true>(s, nullptr, k, v, out, stream, ga);
+    return launch_dw<D, 1, true>(s, q, k, v, out, stream, ga);
   case 2:
-    return launch_dw<D, 2, true>(s, nullptr, k, v, out, stream, ga);
+    return launch_dw<D, 2, true>(s, q, k, v, out, stream, ga);
   case 4:
     if (D == 256 && use_halves(s))
-      return launch_halves<true>(s, nullptr, k, v, out, stream, ga);
-    return launch_dw<D, 4, true>(s, nullptr, k, v, out, stream, ga);
+      return launch_halves<true>(s, q, k, v, out, stream, ga);
+    return launch_dw<D, 4, true>(s, q, k, v, out, stream, ga);
   }
   return hipErrorInvalidValue;
 }
@@ -1356,7 +1149,7 @@ SplitPlan split_plan(const GqaShape &s) {
 template <int D>
 hipError_t launch_split_d(const GqaShape &s, const uint16_t *q, const uint16_t *k,
                           const uint16_t *v, uint16_t *out, void *workspace,
-                          const GatedRows *ga, hipStream_t stream) {
+                          const GateArgs *ga, hipStream_t stream) {
   const SplitPlan p = split_plan(s);
   const unsigned nb = (s.T + BM - 1) / BM;
   const size_t units = (size_t)p.splits * nb * s.Hq;
@@ -1366,21 +1159,21 @@ hipError_t launch_split_d(const GqaShape &s, const uint16_t *q, const uint16_t *
   sa.splits = p.splits;
   hipError_t rc = hipErrorInvalidValue;
   if (p.halves) {
-    rc = launch_halves<false, true>(s, q, k, v, out, stream, NoRows{}, sa);
+    rc = launch_halves<false, true>(s, q, k, v, out, stream, NoArgs{}, sa);
   } else {
     switch (heads_per_wg<D>(s.Hq / s.Hkv)) {
     case 1:
-      rc = launch_dw<D, 1, false, true>(s, q, k, v, out, stream, NoRows{}, sa);
+      rc = launch_dw<D, 1, false, true>(s, q, k, v, out, stream, NoArgs{}, sa);
       break;
     case 2:
-      rc = launch_dw<D, 2, false, true>(s, q, k, v, out, stream, NoRows{}, sa);
+      rc = launch_dw<D, 2, false, true>(s, q, k, v, out, stream, NoArgs{}, sa);
       break;
     case 4:
-      rc = launch_dw<D, 4, false, true>(s, q, k, v, out, stream, NoRows{}, sa);
+      rc = launch_dw<D, 4, false, true>(s, q, k, v, out, stream, NoArgs{}, sa);
       break;
     case 8:
       if constexpr (D == 128)
-        rc = launch_dw<D, 8, false, true>(s, q, k, v, out, stream, NoRows{}, sa);
+        rc = launch_dw<D, 8, false, true>(s, q, k, v, out, stream, NoArgs{}, sa);
       break;
     }
   }
@@ -1390,8 +1183,7 @@ hipError_t launch_split_d(const GqaShape &s, const uint16_t *q, const uint16_t *
   half_t *o = reinterpret_cast<half_t *>(out);
   if (ga)
     hipLaunchKernelGGL((gqa_prefill_merge_kernel<D, true>), grid, dim3(256), 0, stream, sa.ml,
-                       sa.o, o, s.T, s.Hq, nb, p.splits,
-                       reinterpret_cast<const half_t *>(ga->qproj), ga->activated);
+                       sa.o, o, s.T, s.Hq, nb, p.splits, ga->qproj, ga->activated);
   else
     hipLaunchKernelGGL((gqa_prefill_merge_kernel<D, false>), grid, dim3(256), 0, stream, sa.ml,
                        sa.o, o, s.T, s.Hq, nb, p.splits, (const half_t *)nullptr, 0u);
@@ -1410,23 +1202,22 @@ bool prefill_supported(const GqaShape &s) {
 }
 
 bool prefill_gated_supported(const GqaShape &s, unsigned rot) {
-  // One K/V buffer per wave holds the wave's rows, their scales and the
-  // cos/sin table of its 32 tokens.
+  // (the shapes that the call has always taken)
   const unsigned HW = s.D == 256 ? heads_per_wg<256>(s.Hkv ? s.Hq / s.Hkv : 0)
                                  : heads_per_wg<128>(s.Hkv ? s.Hq / s.Hkv : 0);
-  // wave 0's buffer also holds the (1 + w) weights and the cos/sin table
   const size_t need = (size_t)BM * (s.D + 8) * 2 + BM * 4 + (size_t)s.D * 4 +
                       (size_t)BM * (rot / 2) * 4;
   return prefill_supported(s) && HW <= 4 && need <= (size_t)BN * 2 * s.D &&
          rot % 16 == 0 && rot <= s.D;
 }
 
-hipError_t launch_gqa_prefill_gated(const uint16_t *k, const uint16_t *v, uint16_t *out,
-                                    const GqaShape &s, const GatedRows &ga,
-                                    hipStream_t stream) {
+hipError_t launch_gqa_prefill_gated(const uint16_t *q, const uint16_t *k, const uint16_t *v,
+                                    uint16_t *out, const GqaShape &s, const uint16_t *qproj,
+                                    unsigned activated, hipStream_t stream) {
+  const GateArgs ga{reinterpret_cast<const half_t *>(qproj), activated};
   if (s.D == 128)
-    return launch_gated_d<128>(s, k, v, out, ga, stream);
-  return launch_gated_d<256>(s, k, v, out, ga, stream);
+    return launch_gated_d<128>(s, q, k, v, out, ga, stream);
+  return launch_gated_d<256>(s, q, k, v, out, ga, stream);
 }
 
 hipError_t launch_gqa_prefill(const uint16_t *q, const uint16_t *k,
@@ -1439,20 +1230,18 @@ hipError_t launch_gqa_prefill(const uint16_t *q, const uint16_t *k,
 
 bool prefill_split(const GqaShape &s) { return split_plan(s).splits > 1; }
 
-// The partials, then (for the gated call) the normalised query rows.
-size_t prefill_split_partial_bytes(const GqaShape &s) {
+size_t prefill_workspace_bytes(const GqaShape &s) {
   const SplitPlan p = split_plan(s);
   const size_t units = (size_t)p.splits * ((s.T + BM - 1) / BM) * s.Hq;
   return p.splits > 1 ? units * BM * (2 + s.D) * sizeof(float) : 0;
 }
-size_t prefill_workspace_bytes(const GqaShape &s) {
-  const size_t partial = prefill_split_partial_bytes(s);
-  return partial ? partial + (size_t)s.T * s.Hq * s.D * 2 : 0;
-}
 
 hipError_t launch_gqa_prefill_split(const uint16_t *q, const uint16_t *k, const uint16_t *v,
                                     uint16_t *out, void *workspace, const GqaShape &s,
-                                    const GatedRows *ga, hipStream_t stream) {
+                                    const uint16_t *qproj, unsigned activated,
+                                    hipStream_t stream) {
+  const GateArgs gate{reinterpret_cast<const half_t *>(qproj), activated};
+  const GateArgs *ga = qproj ? &gate : nullptr;
   if (s.D == 128)
     return launch_split_d<128>(s, q, k, v, out, workspace, ga, stream);
   return launch_split_d<256>(s, q, k, v, out, workspace, ga, stream);

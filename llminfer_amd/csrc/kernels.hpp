@@ -67,26 +67,25 @@ hipError_t launch_gqa_decode_gated(uint16_t *k, uint16_t *v, uint16_t *out, void
 
 // MFMA flash prefill.
 bool prefill_supported(const GqaShape &s);
-// The gated prefill: the query rows through normRope in the kernel, the
-// output through the sigmoid gate (the keys must already be normRoped into
-// the cache, the values appended).
+// The gated prefill of normalised query rows (which may lie in `out`): the
+// output through the sigmoid gate of qproj's gate halves.
 bool prefill_gated_supported(const GqaShape &s, unsigned rot);
-hipError_t launch_gqa_prefill_gated(const uint16_t *k, const uint16_t *v, uint16_t *out,
-                                    const GqaShape &s, const GatedRows &ga,
-                                    hipStream_t stream);
+hipError_t launch_gqa_prefill_gated(const uint16_t *q, const uint16_t *k, const uint16_t *v,
+                                    uint16_t *out, const GqaShape &s, const uint16_t *qproj,
+                                    unsigned activated, hipStream_t stream);
 hipError_t launch_gqa_prefill(const uint16_t *q, const uint16_t *k,
                               const uint16_t *v, uint16_t *out,
                               const GqaShape &s, hipStream_t stream);
 // A prefill whose grid would leave CUs idle divides its keys over several
 // workgroups a block of rows, with a merge launch after it; it runs where the
-// caller's workspace holds prefill_workspace_bytes. ga: q are the normalised
-// rows (normRope's output) and the merge applies the gate of ga's rows.
+// caller's workspace holds prefill_workspace_bytes. qproj: the merge applies
+// its gates (else null); q may lie in `out`.
 bool prefill_split(const GqaShape &s);
-size_t prefill_split_partial_bytes(const GqaShape &s); // the normalised rows lie behind
 size_t prefill_workspace_bytes(const GqaShape &s);
 hipError_t launch_gqa_prefill_split(const uint16_t *q, const uint16_t *k, const uint16_t *v,
                                     uint16_t *out, void *workspace, const GqaShape &s,
-                                    const GatedRows *ga, hipStream_t stream);
+                                    const uint16_t *qproj, unsigned activated,
+                                    hipStream_t stream);
 
 // Generic fallback for any head_dim <= 512 and any GQA ratio.
 bool generic_supported(const GqaShape &s);
@@ -186,6 +185,15 @@ bool norm_rope_tiled(const RopeShape &s, const void *in, const void *out);
 bool norm_rope_wide_rows(const RopeShape &s);
 hipError_t launch_norm_rope(const uint16_t *in, const float *w, uint16_t *out,
                             const RopeShape &s, hipStream_t stream);
+// A prefill's rows ahead of its attention: normRope of the queries and of the
+// new keys and the copy of `count` value halves, in one launch where the tile
+// kernel takes both shapes, everything is 16-byte aligned and the queries'
+// output lies apart from the keys and values, else in three (the queries'
+// last).
+hipError_t launch_attention_rows(const uint16_t *q, const float *qw, uint16_t *qout,
+                                 const RopeShape &qs, const uint16_t *k, const float *kw,
+                                 uint16_t *kout, const RopeShape &ks, const uint16_t *v,
+                                 uint16_t *vout, unsigned count, hipStream_t stream);
 
 bool sigmoid_mul_vectorised(unsigned count, const void *g, const void *x, const void *o);
 hipError_t launch_sigmoid_mul(const uint16_t *gate, const uint16_t *in, uint16_t *out,

@@ -68,12 +68,12 @@ __device__ __forceinline__ float inv_freq(const RopeFreqs &f, const TileArgs &a,
   return a.rot / 2 <= kArgFreqs ? f.v[i] : rope_inv_freq(a.theta, i, a.rot);
 }
 
+// Tile `block` of the rows (a wave).
 template <bool kNorm>
-__global__ __launch_bounds__(64) void norm_rope_tile(const uint16_t *in,
-                                                     const float *__restrict__ w,
-                                                     uint16_t *out, TileArgs a,
-                                                     RopeFreqs f) {
-  extern __shared__ __align__(16) unsigned char smem[];
+__device__ __forceinline__ void norm_rope_tile_rows(unsigned block, const uint16_t *in,
+                                                    const float *__restrict__ w, uint16_t *out,
+                                                    const TileArgs &a, const RopeFreqs &f,
+                                                    unsigned char *smem) {
   const unsigned lane = threadIdx.x;
   const unsigned pitch = a.D + kPad;
   const unsigned half = a.rot / 2;
@@ -83,7 +83,7 @@ __global__ __launch_bounds__(64) void norm_rope_tile(const uint16_t *in,
   float *wt1 = reinterpret_cast<float *>(rtok + ((a.rw + 1) & ~1u));
   float2 *cs = reinterpret_cast<float2 *>(wt1 + (kNorm ? a.D : 0));
 
-  const unsigned row0 = blockIdx.x * a.rw;
+  const unsigned row0 = block * a.rw;
   const unsigned nrows = min(a.rw, a.rows - row0);
   const unsigned cpr = a.D / 8; // 16-byte chunks per row
   // Lane l owns chunks l, l + 64, ... of the tile, row-major; (r, col) of
@@ -247,6 +247,37 @@ __global__ __launch_bounds__(64) void norm_rope_tile(const uint16_t *in,
       }
     }
   }
+}
+
+template <bool kNorm>
+__global__ __launch_bounds__(64) void norm_rope_tile(const uint16_t *in,
+                                                     const float *__restrict__ w,
+                                                     uint16_t *out, TileArgs a,
+                                                     RopeFreqs f) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  norm_rope_tile_rows<kNorm>(blockIdx.x, in, w, out, a, f, smem);
+}
+
+// A prefill's rows in one launch: the query tiles, the key tiles, then the
+// value rows, 8 KB a wave. Each alone is latency (8 us for 333 tokens of 16
+// query or 4 key heads, 3 us for the values), so together they take the time
+// of one (9 us).
+constexpr unsigned kCopyVectors = 8 * 64; // 16-byte vectors a wave copies
+
+__global__ __launch_bounds__(64) void attention_rows(
+    const uint16_t *q, const float *__restrict__ qw, uint16_t *qout, TileArgs qa, unsigned qtiles,
+    const uint16_t *k, const float *__restrict__ kw, uint16_t *kout, TileArgs ka, unsigned ktiles,
+    const uint4_t *v, uint4_t *vout, unsigned vectors, RopeFreqs f) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  if (blockIdx.x < qtiles)
+    return norm_rope_tile_rows<true>(blockIdx.x, q, qw, qout, qa, f, smem);
+  if (blockIdx.x < qtiles + ktiles)
+    return norm_rope_tile_rows<true>(blockIdx.x - qtiles, k, kw, kout, ka, f, smem);
+  const unsigned i0 = (blockIdx.x - qtiles - ktiles) * kCopyVectors + threadIdx.x;
+#pragma unroll
+  for (unsigned u = 0; u < kCopyVectors / 64; ++u)
+    if (i0 + 64 * u < vectors)
+      vout[i0 + 64 * u] = v[i0 + 64 * u];
 }
 
 // One thread per row: the reference kernel's structure, for any alignment.
@@ -456,6 +487,36 @@ hipError_t launch_norm_rope(const uint16_t *in, const float *w, uint16_t *out,
     else
       hipLaunchKernelGGL(norm_rope_rows<false>, grid, dim3(256), 0, stream, in, w, out, a, f);
   }
+  return hipGetLastError();
+}
+
+hipError_t launch_attention_rows(const uint16_t *q, const float *qw, uint16_t *qout,
+                                 const RopeShape &qs, const uint16_t *k, const float *kw,
+                                 uint16_t *kout, const RopeShape &ks, const uint16_t *v,
+                                 uint16_t *vout, unsigned count, hipStream_t stream) {
+  auto apart = [&](const void *in, size_t halves) { // from the queries' output
+    const uintptr_t a = (uintptr_t)qout, b = (uintptr_t)in;
+    return a + 2 * (size_t)qs.rows * qs.D <= b || b + 2 * halves <= a;
+  };
+  if (!apart(k, (size_t)ks.rows * ks.stride) || !apart(v, count) ||
+      !norm_rope_tiled(qs, q, qout) || !norm_rope_tiled(ks, k, kout) || !qs.norm || !ks.norm ||
+      qs.theta != ks.theta || qs.rot != ks.rot || count % 8 || !aligned16(v) || !aligned16(vout)) {
+    hipError_t e = launch_norm_rope(k, kw, kout, ks, stream);
+    if (e == hipSuccess)
+      e = launch_cache_append(v, vout, count, 0, stream);
+    return e == hipSuccess ? launch_norm_rope(q, qw, qout, qs, stream) : e;
+  }
+  const TilePlan qp = plan_tile(qs), kp = plan_tile(ks);
+  const TileArgs qa{qs.rows, qs.heads, qs.D, qs.rot, qs.stride, qs.past, qs.out_row0,
+                    qp.rw, qp.maxtok, qs.eps, qs.theta};
+  const TileArgs ka{ks.rows, ks.heads, ks.D, ks.rot, ks.stride, ks.past, ks.out_row0,
+                    kp.rw, kp.maxtok, ks.eps, ks.theta};
+  const unsigned qtiles = (qs.rows + qp.rw - 1) / qp.rw, ktiles = (ks.rows + kp.rw - 1) / kp.rw;
+  const unsigned vectors = count / 8, copies = (vectors + kCopyVectors - 1) / kCopyVectors;
+  hipLaunchKernelGGL(attention_rows, dim3(qtiles + ktiles + copies), dim3(64),
+                     qp.lds > kp.lds ? qp.lds : kp.lds, stream, q, qw, qout, qa, qtiles, k, kw,
+                     kout, ka, ktiles, reinterpret_cast<const uint4_t *>(v),
+                     reinterpret_cast<uint4_t *>(vout), vectors, host_freqs(qs.theta, qs.rot));
   return hipGetLastError();
 }
 
