@@ -75,19 +75,27 @@ __global__ __launch_bounds__(256) void elementwise_kernel(const uint16_t *__rest
   }
 }
 
+// Piece i of the view, kPiece halves along its innermost axis. Bound by memory
+// and, a half a lane, by the index arithmetic of its three axes, which a piece
+// of eight shares (the three views of a DeltaNet layer's 1024 x 8192 halves:
+// 22 -> 10 us together).
+template <unsigned kPiece>
 __global__ __launch_bounds__(256) void copy_view_kernel(const uint16_t *__restrict__ src,
                                                         uint16_t *__restrict__ out,
                                                         HalfViewParams p) {
   const unsigned i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= p.count)
+  if (i >= p.count / kPiece)
     return;
-  unsigned rest = i, offset = p.offset;
+  unsigned rest = i * kPiece, offset = p.offset;
 #pragma unroll
   for (int d = 2; d >= 0; --d) {
     offset += (rest % p.dims[d]) * p.strides[d];
     rest /= p.dims[d];
   }
-  out[i] = src[offset];
+  if constexpr (kPiece == 8)
+    reinterpret_cast<uint4_t *>(out)[i] = *reinterpret_cast<const uint4_t *>(src + offset);
+  else
+    out[i] = src[offset];
 }
 
 // ------------------------------------------------------------- linearF16
@@ -300,8 +308,19 @@ hipError_t launch_elementwise(ElementwiseKind kind, const uint16_t *a, const uin
 
 hipError_t launch_copy_half_view(const uint16_t *src, uint16_t *out, const HalfViewParams &p,
                                  hipStream_t stream) {
-  hipLaunchKernelGGL(copy_view_kernel, dim3((p.count + 255) / 256), dim3(256), 0, stream, src,
-                     out, p);
+  // Eight halves a lane where every piece is whole, consecutive and 16-byte
+  // aligned on both sides: an innermost extent of whole pieces, the other axes'
+  // strides of whole pieces wherever they are stepped along.
+  const bool pieces =
+      p.strides[2] == 1 && p.dims[2] % 8 == 0 && (p.dims[1] == 1 || p.strides[1] % 8 == 0) &&
+      (p.dims[0] == 1 || p.strides[0] % 8 == 0) &&
+      (reinterpret_cast<uintptr_t>(src + p.offset) | reinterpret_cast<uintptr_t>(out)) % 16 == 0;
+  if (pieces)
+    hipLaunchKernelGGL(copy_view_kernel<8>, dim3((p.count / 8 + 255) / 256), dim3(256), 0, stream,
+                       src, out, p);
+  else
+    hipLaunchKernelGGL(copy_view_kernel<1>, dim3((p.count + 255) / 256), dim3(256), 0, stream,
+                       src, out, p);
   return hipGetLastError();
 }
 

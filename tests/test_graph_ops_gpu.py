@@ -78,6 +78,24 @@ def test_copy_half_view_bit_exact(gpu, shape, axis, begin, length):
     assert np.array_equal(_host_u16(out).reshape(view.shape), np.ascontiguousarray(view))
 
 
+# Pieces of eight (whole, strided, an outer axis of one), and each reason to go
+# a half at a time: begin, extent, stride or buffer off by less than a piece.
+@pytest.mark.parametrize("shape,begin,length,shift", [
+    ((1, 1, 8), 0, 8, 0), ((3, 5, 64), 8, 24, 0), ((1, 37, 2056), 2048, 8, 0),
+    ((2, 300, 64), 32, 32, 0), ((3, 5, 64), 4, 24, 0), ((3, 5, 64), 8, 20, 0),
+    ((3, 5, 60), 8, 24, 0), ((3, 5, 64), 8, 24, 1)])
+def test_copy_half_view_pieces_and_halves(gpu, shape, begin, length, shift):
+    src = np.random.default_rng(2).integers(0, 0x7C00, shape).astype(np.uint16)
+    view = src[:, :, begin:begin + length]
+    strides = [s // 2 for s in view.strides]
+    guard = torch.full((view.size + shift + 8,), 3.0, dtype=torch.float16, device=gpu)
+    out = guard[shift:shift + view.size]
+    ops.copy_half_view(_u16_dev(src, gpu), out, view.shape, strides, begin)
+    torch.cuda.synchronize()
+    assert np.array_equal(_host_u16(out).reshape(view.shape), np.ascontiguousarray(view))
+    assert bool((guard[:shift] == 3).all()) and bool((guard[shift + view.size:] == 3).all())
+
+
 @pytest.mark.parametrize("tokens,k,columns", [(1, 2560, 300), (3, 70, 33), (9, 64, 256),
                                               (17, 129, 513), (1, 1, 5)])
 def test_linear_f16_bit_exact(gpu, tokens, k, columns):
