@@ -44,6 +44,29 @@ def test_causal_conv(gpu, T, C, k, silu):
         assert np.array_equal(torch_to_u16(ht), href)
 
 
+# Two channels a lane and eight tokens (k = 4, several tokens, whole words) at
+# its edges: histories longer than the call, a block's last and next token, a
+# workgroup's last pair; an odd row length and a misaligned input (shift) stay
+# with a lane a channel.
+@pytest.mark.parametrize("T,C,silu,shift", [
+    (2, 2, True, 0), (3, 512, True, 0), (4, 510, False, 0), (8, 514, True, 0),
+    (9, 1026, True, 0), (17, 512, True, 0), (9, 511, True, 0), (9, 512, True, 1)])
+def test_causal_conv_pairs(gpu, T, C, silu, shift):
+    rng = np.random.default_rng(T * 37 + C)
+    x, w, h = _f16(rng, (T, C), 3.0), _f16(rng, (C, 4), 0.5), _f16(rng, (C, 3))
+    print(f"causalConv pairs T={T} C={C} silu={silu} shift={shift}", flush=True)
+    xt = torch.empty(T * C + shift, dtype=torch.float16, device=gpu)[shift:].view(T, C)
+    xt.copy_(u16_to_torch(x))
+    ht = u16_to_torch(h)
+    out = torch.empty(T, C, dtype=torch.float16, device=gpu)
+    ops.causal_conv(xt, u16_to_torch(w), ht, out, silu)
+    torch.cuda.synchronize()
+    href = h.copy()
+    ref = oracle.causal_conv(x, w, href, silu)
+    assert np.array_equal(torch_to_u16(out), ref)
+    assert np.array_equal(torch_to_u16(ht), href)
+
+
 def test_causal_conv_split_calls_carry_history(gpu):
     rng = np.random.default_rng(5)
     T, C, k = 40, 256, 4
