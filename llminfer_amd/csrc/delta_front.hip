@@ -16,7 +16,7 @@
 // sequence) after reading, so no thread races it. Loads and stores are
 // coalesced across the channels of a wave.
 //
-// l2NormF32: one wave per 16 rows; the rows are staged in LDS with 16-byte
+// l2NormF32: one wave per 4 or 8 rows; the rows are staged in LDS with 16-byte
 // coalesced loads, lane r sums row r in index order (the reference's fma
 // chain), and the fp32 outputs leave as 16-byte stores. Other widths and
 // unaligned buffers take a thread per row.
@@ -36,7 +36,13 @@ namespace {
 
 constexpr unsigned kConvBlock = 16; // tokens per thread
 constexpr unsigned kMaxKernel = 8;  // filter taps supported (history 7)
-constexpr unsigned kL2Rows = 16;    // l2NormF32 rows per wave (16K rows fill 1024 waves)
+// Rows a wave of the two tile kernels. A call of few rows is bound by one wave's
+// own latency, which grows with its rows, and a call of many by memory: width
+// 128, rows a wave 16 / 8 / 4 in us, l2NormF32 4.1 / 3.2 / 2.8 at 32 rows,
+// 5.0 / 4.2 / 3.9 at 8192, 5.8 / 5.0 / 5.1 at 16384, 7.1 / 7.0 / 7.7 at 32768;
+// gatedRmsNorm 6.8 / 4.6 / 3.5, 7.8 / 5.9 / 5.3, 8.9 / 7.6 / 7.2, 12.1 / 11.5 /
+// 11.6. So four up to kFewRows, eight past it.
+constexpr unsigned kFewRows = 16384;
 
 __global__ __launch_bounds__(256) void causal_conv_kernel(
     const uint16_t *__restrict__ in, const uint16_t *__restrict__ w, uint16_t *hist,
@@ -244,14 +250,15 @@ __device__ __forceinline__ float l2_factor(float sum, float eps, float scale) {
   return l2_row_factor(sum, eps, scale);
 }
 
-// Rows of `width` (a multiple of 8, <= 256) halves, kL2Rows per wave.
+// Rows of `width` (a multiple of 8, <= 256) halves, kRows per wave.
+template <unsigned kRows>
 __global__ __launch_bounds__(64) void l2_norm_tile(const uint16_t *__restrict__ in,
                                                    float *__restrict__ out, unsigned rows,
                                                    unsigned width, float eps, float scale) {
-  __shared__ __align__(16) uint16_t tile[kL2Rows * (256 + 8)];
-  __shared__ float fac[kL2Rows];
+  __shared__ __align__(16) uint16_t tile[kRows * (256 + 8)];
+  __shared__ float fac[kRows];
   const unsigned lane = threadIdx.x, pitch = width + 8, cpr = width / 8;
-  const unsigned row0 = blockIdx.x * kL2Rows, nrows = min(kL2Rows, rows - row0);
+  const unsigned row0 = blockIdx.x * kRows, nrows = min(kRows, rows - row0);
   const unsigned chunks = nrows * cpr;
   for (unsigned c = lane; c < chunks; c += 64) {
     unsigned r = c / cpr, col = c - r * cpr;
@@ -333,14 +340,14 @@ __global__ __launch_bounds__(256) void gated_rms_norm_rows(const uint16_t *__res
   }
 }
 
-// gatedRmsNorm (Reference.metal:228-259): kL2Rows rows of `width` (a
+// gatedRmsNorm (Reference.metal:228-259): kRows rows of `width` (a
 // multiple of 8, <= 256) per wave, staged in LDS like l2_norm_tile; out =
 // fp16(fp16(x * scale) * w * g) with g = silu(gate) for an fp16 gate (an
 // estimate that the margin test accepts, else exact) or the fp32 gate.
 // kQuant: the stored fp16 rows also quantized (quantizeActivation's
 // expressions over the flattened rows: 32-wide groups, four lanes' chunks
 // of eight, width a multiple of 32) into qout, scales and the invalid flag.
-template <bool kActivated, bool kQuant>
+template <bool kActivated, bool kQuant, unsigned kRows>
 __global__ __launch_bounds__(64) void gated_rms_norm_tile(const uint16_t *__restrict__ in,
                                                           const void *__restrict__ gate,
                                                           const float *__restrict__ w,
@@ -349,10 +356,10 @@ __global__ __launch_bounds__(64) void gated_rms_norm_tile(const uint16_t *__rest
                                                           float eps, int8_t *__restrict__ qout,
                                                           float *__restrict__ scales,
                                                           unsigned *invalid) {
-  __shared__ __align__(16) uint16_t tile[kL2Rows * (256 + 8)];
-  __shared__ float fac[kL2Rows];
+  __shared__ __align__(16) uint16_t tile[kRows * (256 + 8)];
+  __shared__ float fac[kRows];
   const unsigned lane = threadIdx.x, pitch = width + 8, cpr = width / 8;
-  const unsigned row0 = blockIdx.x * kL2Rows, nrows = min(kL2Rows, rows - row0);
+  const unsigned row0 = blockIdx.x * kRows, nrows = min(kRows, rows - row0);
   const unsigned chunks = nrows * cpr;
   for (unsigned c = lane; c < chunks; c += 64) {
     unsigned r = c / cpr, col = c - r * cpr;
@@ -487,9 +494,12 @@ hipError_t launch_l2_norm(const uint16_t *in, float *out, unsigned rows, unsigne
                           float eps, float scale, hipStream_t stream) {
   if (rows == 0 || width == 0)
     return hipSuccess;
-  if (l2_norm_tiled(width, in, out))
-    hipLaunchKernelGGL(l2_norm_tile, dim3((rows + kL2Rows - 1) / kL2Rows), dim3(64), 0, stream, in, out,
-                       rows, width, eps, scale);
+  if (l2_norm_tiled(width, in, out) && rows <= kFewRows)
+    hipLaunchKernelGGL(l2_norm_tile<4>, dim3((rows + 3) / 4), dim3(64), 0, stream, in, out, rows,
+                       width, eps, scale);
+  else if (l2_norm_tiled(width, in, out))
+    hipLaunchKernelGGL(l2_norm_tile<8>, dim3((rows + 7) / 8), dim3(64), 0, stream, in, out, rows,
+                       width, eps, scale);
   else
     hipLaunchKernelGGL(l2_norm_rows, dim3((rows + 255) / 256), dim3(256), 0, stream, in, out,
                        rows, width, eps, scale);
@@ -498,6 +508,20 @@ hipError_t launch_l2_norm(const uint16_t *in, float *out, unsigned rows, unsigne
 
 bool gated_rms_norm_tiled(unsigned width, const void *in, const void *gate, const void *out) {
   return width % 8 == 0 && width <= 256 && aligned16(in) && aligned16(gate) && aligned16(out);
+}
+
+template <bool kActivated, bool kQuant>
+static void launch_gated_tile(const uint16_t *in, const void *gate, const float *w, uint16_t *out,
+                              int8_t *q, float *scales, unsigned *invalid, unsigned rows,
+                              unsigned width, float eps, hipStream_t stream) {
+  if (rows <= kFewRows)
+    hipLaunchKernelGGL((gated_rms_norm_tile<kActivated, kQuant, 4>), dim3((rows + 3) / 4),
+                       dim3(64), 0, stream, in, gate, w, out, rows, width, eps, q, scales,
+                       invalid);
+  else
+    hipLaunchKernelGGL((gated_rms_norm_tile<kActivated, kQuant, 8>), dim3((rows + 7) / 8),
+                       dim3(64), 0, stream, in, gate, w, out, rows, width, eps, q, scales,
+                       invalid);
 }
 
 hipError_t launch_gated_rms_norm(const uint16_t *in, const void *gate, bool activated,
@@ -515,13 +539,12 @@ hipError_t launch_gated_rms_norm(const uint16_t *in, const void *gate, bool acti
                          rows, width, eps);
     return hipGetLastError();
   }
-  dim3 grid((rows + kL2Rows - 1) / kL2Rows);
   if (activated)
-    hipLaunchKernelGGL((gated_rms_norm_tile<true, false>), grid, dim3(64), 0, stream, in, gate,
-                       w, out, rows, width, eps, nullptr, nullptr, nullptr);
+    launch_gated_tile<true, false>(in, gate, w, out, nullptr, nullptr, nullptr, rows, width, eps,
+                                   stream);
   else
-    hipLaunchKernelGGL((gated_rms_norm_tile<false, false>), grid, dim3(64), 0, stream, in, gate,
-                       w, out, rows, width, eps, nullptr, nullptr, nullptr);
+    launch_gated_tile<false, false>(in, gate, w, out, nullptr, nullptr, nullptr, rows, width, eps,
+                                    stream);
   return hipGetLastError();
 }
 
@@ -536,9 +559,7 @@ hipError_t launch_gated_rms_norm_quantize(const uint16_t *in, const float *gate,
                                           float eps, hipStream_t stream) {
   if (rows == 0)
     return hipSuccess;
-  hipLaunchKernelGGL((gated_rms_norm_tile<true, true>), dim3((rows + kL2Rows - 1) / kL2Rows),
-                     dim3(64), 0, stream, in, gate, w, out, rows, width, eps, q, scales,
-                     invalid);
+  launch_gated_tile<true, true>(in, gate, w, out, q, scales, invalid, rows, width, eps, stream);
   return hipGetLastError();
 }
 

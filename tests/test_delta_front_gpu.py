@@ -144,6 +144,29 @@ def test_gate_beta_every_fp16_value(gpu):
     assert np.array_equal(beta.cpu().numpy().view(np.uint32), rb.view(np.uint32))
 
 
+# Four rows a wave up to 16384 rows, eight past it: ragged last waves, either
+# side of the rule, and the widest row.
+@pytest.mark.parametrize("rows,width", [(1, 256), (5, 40), (7, 128), (16383, 8), (16384, 8),
+                                        (16385, 8), (16391, 256)])
+def test_row_norms_rows_a_wave(gpu, rows, width):
+    rng = np.random.default_rng(rows * 3 + width)
+    x, g = _f16(rng, (rows, width)), _f16(rng, (rows, width), 2.0)
+    w = (1.0 + 0.1 * rng.standard_normal(width)).astype(np.float32)
+    print(f"row norms rows={rows} width={width}", flush=True)
+    xt, wt = u16_to_torch(x), torch.from_numpy(w).to(gpu)
+    l2 = torch.empty(rows, width, dtype=torch.float32, device=gpu)
+    ops.l2_norm(xt, l2, width, 1e-6, 0.5)
+    plain, activated = torch.empty_like(xt), torch.empty_like(xt)
+    ops.gated_rms_norm(xt, u16_to_torch(g), wt, plain)
+    gf = oracle.f16_to_f32(g)
+    ops.gated_rms_norm(xt, torch.from_numpy(gf).to(gpu), wt, activated)
+    torch.cuda.synchronize()
+    assert np.array_equal(l2.cpu().numpy().view(np.uint32),
+                          oracle.l2norm_f32(x, width, 1e-6, 0.5).view(np.uint32))
+    assert np.array_equal(torch_to_u16(plain), oracle.gated_rms_norm(x, g, w))
+    assert np.array_equal(torch_to_u16(activated), oracle.gated_rms_norm(x, gf, w))
+
+
 @pytest.mark.parametrize("rows,width,activated", [(1024 * 32, 128, False), (32, 128, False),
                                                   (1000, 128, True), (45, 256, False),
                                                   (7, 64, True),
