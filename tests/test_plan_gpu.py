@@ -199,6 +199,38 @@ def test_session_rejects_bad_steps_and_resets(gpu):
     assert np.array_equal(session.step(TOKENS[:4]).logits, a)
 
 
+def test_session_steps_do_not_depend_on_the_step_before(gpu):
+    """The next one-row step is lowered behind a step: taken at the same
+    logits mode, passed over at another, after several rows or a reset, absent
+    at the capacity. One row's logits are the same bits in every mode."""
+    c = small_qwen35()
+    weights = device_weights(_small_weights(c, 5), gpu)
+    same = ModelSession(c, weights, 24, True, gpu)
+    mixed = ModelSession(c, weights, 24, True, gpu)
+    chunks = [list(range(10, 17)), [3], [4], [5], [6], [7], list(range(30, 36)), [8], [9], [1],
+              [2], [11], [12]]
+    modes = ["none", "last", "all", "all", "none", "last", "last", "last", "all", "last", "none",
+             "last", "last"]
+    assert sum(map(len, chunks)) == 24
+    for turn in range(2):
+        for chunk, mode in zip(chunks, modes):
+            want, got = same.step(chunk, "last").logits, mixed.step(chunk, mode).logits
+            if mode != "none":
+                assert np.array_equal(got[-1:], want), (turn, chunk, mode)
+        for a, b in zip(same.states, mixed.states):
+            assert _same_state(a, b)
+        for session in (same, mixed):
+            with pytest.raises(ValueError):
+                session.step([1])
+            session.reset()
+        # a step right after the reset's first, at the position of an old plan
+        same.step([3])
+        mixed.step([3], "all")
+        assert np.array_equal(same.step([4]).logits, mixed.step([4]).logits)
+        same.reset()
+        mixed.reset()
+
+
 def test_qwen35_4b_decode_step(gpu):
     """Qwen3.5-4B (32 layers, random W8A8 weights of its shapes): a 64-token
     prefill and a decode step through the session equal, bit for bit, the

@@ -124,6 +124,27 @@ def test_linear_shard_writes_only_its_columns(gpu):
     assert np.all(got2[:, :30] == 0x4700) and np.all(got2[:, 78:] == 0x4700)
 
 
+# The matrix kernel's tile (32 x 32) and steps (eight groups, one a wave) at
+# their edges, several tiles each way, and its smallest call; what lies beside
+# the written columns and rows stays as it was.
+@pytest.mark.parametrize("rows,columns,groups", [
+    (2, 1, 1), (2, 31, 7), (31, 32, 8), (32, 33, 9), (33, 31, 16), (33, 65, 17), (65, 64, 24),
+    (97, 97, 25)])
+def test_linear_gemm_tile_edges(gpu, rows, columns, groups):
+    print(f"linearW8A8Gemm edges rows={rows} columns={columns} groups={groups}", flush=True)
+    xq, xs, w, ws = _case(7000 + rows + columns + groups, rows, columns, groups)
+    # rows of the output past the call's, columns either side of it
+    out = torch.full((rows + 1, columns + 3), 3.0, dtype=torch.float16, device=gpu)
+    ops.linear_w8a8(_dev(xq, gpu), _dev(xs, gpu), _dev(w, gpu), _u16_dev(ws, gpu), out[:rows],
+                    first_row=1)
+    torch.cuda.synchronize()
+    got = _host_u16(out)
+    assert np.array_equal(got[:rows, 1:1 + columns], oracle.linear_w8a8(xq, xs, w, ws))
+    rest = out.clone()
+    rest[:rows, 1:1 + columns] = 3.0
+    assert bool((rest == 3.0).all())
+
+
 @pytest.mark.parametrize("rows,groups", [(1, 20), (1, 160), (6, 20), (20, 20), (40, 160)])
 @pytest.mark.parametrize("epilogue", [1, 2, 3, 4, 5, 6])
 def test_linear_epilogues_bit_exact(gpu, rows, groups, epilogue):
