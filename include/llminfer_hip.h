@@ -346,8 +346,10 @@ LLMI_HIP_API int llmi_hip_kv_append_causal_gqa_noalloc(const uint16_t *q,
  * k), llmi_hip_cache_append, llmi_hip_causal_gqa and llmi_hip_sigmoid_mul
  * run in that order. T == 1 is one decode launch (plus its merge) that does
  * all of it; T > 1 normRopes q into out and K into the cache and appends V
- * (one launch), then runs the MFMA prefill of out's rows with the gate in its
- * output store, or in its merge where it divides its keys. Workspace:
+ * (one launch; one each, K, V, q, where a buffer is not 16-byte aligned or one
+ * of these inputs lies in the rows that another one's launch writes), then runs
+ * the MFMA prefill of out's rows with the gate in its output store, or in its
+ * merge where it divides its keys. Workspace:
  * llmi_hip_gqa_workspace_bytes(p), as for llmi_hip_causal_gqa (the bits are
  * those of that call with as large a workspace).
  * Supported: d 128 or 256, Hq/Hkv 2 or 4 (decode) or <= 4 (prefill),

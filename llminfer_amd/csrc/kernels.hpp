@@ -187,9 +187,9 @@ hipError_t launch_norm_rope(const uint16_t *in, const float *w, uint16_t *out,
                             const RopeShape &s, hipStream_t stream);
 // A prefill's rows ahead of its attention: normRope of the queries and of the
 // new keys and the copy of `count` value halves, in one launch where the tile
-// kernel takes both shapes, everything is 16-byte aligned and the queries'
-// output lies apart from the keys and values, else in three (the queries'
-// last).
+// kernel takes both shapes, everything is 16-byte aligned and each input lies
+// apart from the other parts' outputs, else in three: the keys', the values',
+// the queries'.
 hipError_t launch_attention_rows(const uint16_t *q, const float *qw, uint16_t *qout,
                                  const RopeShape &qs, const uint16_t *k, const float *kw,
                                  uint16_t *kout, const RopeShape &ks, const uint16_t *v,

@@ -494,11 +494,18 @@ hipError_t launch_attention_rows(const uint16_t *q, const float *qw, uint16_t *q
                                  const RopeShape &qs, const uint16_t *k, const float *kw,
                                  uint16_t *kout, const RopeShape &ks, const uint16_t *v,
                                  uint16_t *vout, unsigned count, hipStream_t stream) {
-  auto apart = [&](const void *in, size_t halves) { // from the queries' output
-    const uintptr_t a = (uintptr_t)qout, b = (uintptr_t)in;
-    return a + 2 * (size_t)qs.rows * qs.D <= b || b + 2 * halves <= a;
+  // One launch runs its parts in no order: each part's input must lie apart
+  // from what the others write (keys staged in the value cache's new rows are
+  // read before the values are appended only where the launches are separate).
+  auto apart = [](const void *in, size_t halves, const void *out, size_t outHalves) {
+    const uintptr_t a = (uintptr_t)in, b = (uintptr_t)out;
+    return a + 2 * halves <= b || b + 2 * outHalves <= a;
   };
-  if (!apart(k, (size_t)ks.rows * ks.stride) || !apart(v, count) ||
+  const size_t nq = (size_t)qs.rows * qs.stride, nk = (size_t)ks.rows * ks.stride;
+  const size_t nqo = (size_t)qs.rows * qs.D, nko = (size_t)ks.rows * ks.D;
+  const uint16_t *krows = kout + (size_t)ks.out_row0 * ks.D;
+  if (!apart(k, nk, qout, nqo) || !apart(k, nk, vout, count) || !apart(v, count, qout, nqo) ||
+      !apart(v, count, krows, nko) || !apart(q, nq, krows, nko) || !apart(q, nq, vout, count) ||
       !norm_rope_tiled(qs, q, qout) || !norm_rope_tiled(ks, k, kout) || !qs.norm || !ks.norm ||
       qs.theta != ks.theta || qs.rot != ks.rot || count % 8 || !aligned16(v) || !aligned16(vout)) {
     hipError_t e = launch_norm_rope(k, kw, kout, ks, stream);

@@ -1,0 +1,190 @@
+// The host code of libllminfer_hip.so without a GPU: this program defines the
+// HIP runtime calls that the library makes, so device memory is host memory
+// (filled with its 16-bit index), copies are copies, and kernel launches are
+// recorded by name and not run. Each command prints lines of
+// "what name name ..." (tests/test_host_path.py).
+#include "llminfer_hip.h"
+
+#include <hip/hip_runtime_api.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <string>
+#include <vector>
+#include <xmmintrin.h>
+
+namespace {
+// (made on first use: the library registers its kernels before main)
+std::map<const void *, std::string> &kernels() {
+  static std::map<const void *, std::string> m;
+  return m;
+}
+std::vector<std::string> launches;
+size_t largest = SIZE_MAX; // allocations above it fail
+hipError_t last = hipSuccess;
+
+// Kernels live in unnamed namespaces: the name follows its length.
+std::string base_name(const char *mangled) {
+  const char *at = strstr(mangled, "_GLOBAL__N_1");
+  if (!at)
+    return mangled;
+  char *name;
+  const long n = strtol(at + 12, &name, 10);
+  return std::string(name, n);
+}
+} // namespace
+
+extern "C" {
+void **__hipRegisterFatBinary(const void *) {
+  static void *handle;
+  return &handle;
+}
+void __hipUnregisterFatBinary(void **) {}
+void __hipRegisterFunction(void **, const void *host, char *, const char *name, unsigned, void *,
+                           void *, void *, void *, int *) {
+  kernels()[host] = base_name(name);
+}
+void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
+
+static thread_local struct {
+  dim3 grid, block;
+  size_t lds;
+  hipStream_t stream;
+} config;
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, hipStream_t s) {
+  config = {g, b, lds, s};
+  return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, hipStream_t *s) {
+  *g = config.grid, *b = config.block, *lds = config.lds, *s = config.stream;
+  return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **, size_t, hipStream_t) {
+  launches.push_back(kernels()[f]);
+  return hipSuccess;
+}
+hipError_t hipMalloc(void **p, size_t n) {
+  if (n > largest)
+    return last = hipErrorOutOfMemory;
+  *p = aligned_alloc(256, (n + 255) / 256 * 256);
+  for (size_t i = 0; i < n / 2; ++i)
+    static_cast<uint16_t *>(*p)[i] = (uint16_t)i;
+  return hipSuccess;
+}
+hipError_t hipFree(void *p) {
+  free(p);
+  return hipSuccess;
+}
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+  *p = malloc(n);
+  return hipSuccess;
+}
+hipError_t hipHostFree(void *p) {
+  free(p);
+  return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) {
+  memcpy(d, s, n);
+  return hipSuccess;
+}
+hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t) {
+  memset(d, v, n);
+  return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipGetLastError() {
+  const hipError_t e = last;
+  last = hipSuccess;
+  return e;
+}
+const char *hipGetErrorString(hipError_t) { return "error"; }
+hipError_t hipGetDevice(int *d) {
+  *d = 0;
+  return hipSuccess;
+}
+hipError_t hipGetDeviceCount(int *n) {
+  *n = 1;
+  return hipSuccess;
+}
+hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) {
+  *v = 256;
+  return hipSuccess;
+}
+hipError_t hipGetDeviceProperties(hipDeviceProp_t *p, int) { // (hipGetDevicePropertiesR0600)
+  memset(p, 0, sizeof *p);
+  strcpy(p->gcnArchName, "gfx950");
+  p->multiProcessorCount = 256;
+  return hipSuccess;
+}
+hipError_t hipGetSymbolAddress(void **p, const void *) {
+  static unsigned char array[LLMI_HIP_NOALLOC_SCRATCH_BYTES];
+  *p = array;
+  return hipSuccess;
+}
+hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *, int, size_t) {
+  *n = 2;
+  return hipSuccess;
+}
+}
+
+namespace {
+
+void flush_launches(const char *what) {
+  printf("%s", what);
+  for (const std::string &n : launches)
+    printf(" %s", n.c_str());
+  printf("\n");
+  launches.clear();
+}
+
+template <typename P> void names(int op, const P &p) {
+  printf("names");
+  for (unsigned i = 0, n = llmi_hip_dispatch_count(op, &p); i < n; ++i)
+    printf(" %s", llmi_hip_kernel_name(op, &p, i));
+  printf("\n");
+}
+
+// gated T past q_heads kv_heads head_dim rotary place: where the projected
+// keys or values lie ("apart", or in an output of the call).
+int gated(char **a) {
+  const GqaParams p{(unsigned)atoi(a[0]), (unsigned)atoi(a[2]), (unsigned)atoi(a[3]),
+                    (unsigned)atoi(a[4]), (unsigned)atoi(a[1])};
+  const std::string place = a[6];
+  const size_t q = (size_t)p.tokens * p.queryHeads * p.headDim,
+               row = (size_t)p.kvHeads * p.headDim, past = p.past * row, kv = p.tokens * row;
+  void *qp, *kp, *vp, *kc, *vc, *out, *ws, *w;
+  const size_t bytes = llmi_hip_gqa_workspace_bytes(p);
+  for (auto [to, n] : {std::pair{&qp, 4 * q}, {&kp, 2 * kv + 16}, {&vp, 2 * kv + 16},
+                       {&kc, 2 * (past + kv)}, {&vc, 2 * (past + kv)}, {&out, 2 * q},
+                       {&ws, bytes}, {&w, size_t{4} * p.headDim}})
+    if (hipMalloc(to, n) != hipSuccess)
+      return 1;
+  auto u16 = [](void *x) { return static_cast<uint16_t *>(x); };
+  uint16_t *k = u16(kp), *v = u16(vp);
+  if (place == "keys_in_values")
+    k = u16(vc) + past;
+  else if (place == "values_in_keys")
+    v = u16(kc) + past;
+  else if (place == "keys_in_output")
+    k = u16(out);
+  else if (place == "keys_unaligned")
+    k += 1;
+  launches.clear();
+  const int rc = llmi_hip_gated_attention(u16(qp), k, v, (float *)w, (float *)w, u16(kc), u16(vc),
+                                          u16(out), p, atoi(a[5]), 1e-6f, 1e7f, ws, bytes, nullptr);
+  printf("status %d\n", rc);
+  flush_launches("launches");
+  names(LLMI_HIP_OP_GATED_ATTENTION, p);
+  return 0;
+}
+
+} // namespace
+
+int main(int argc, char **argv) {
+  const std::string command = argc > 1 ? argv[1] : "";
+  if (command == "gated" && argc == 9)
+    return gated(argv + 2);
+  return 2;
+}

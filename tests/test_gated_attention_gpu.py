@@ -99,6 +99,39 @@ def test_divided_block_equals_the_unfused_ops(gpu, T, past, shape, rot):
     assert _lib.load().llmi_hip_gqa_workspace_bytes(_lib.GqaParams(T, hq, hkv, d, past)) > 0
 
 
+@pytest.mark.parametrize("place", ["keys_in_values", "keys_in_output", "unaligned"])
+@pytest.mark.parametrize("T,past", [(333, 0), (40, 700)])
+def test_block_whose_rows_lie_in_its_outputs(gpu, place, T, past):
+    """The projected keys staged in the value cache's new rows or in the
+    output, and keys and values that are not 16-byte aligned: the rows run
+    as separate launches, with the bits of rows that lie apart."""
+    hq, hkv, d = 16, 4, 256
+    print(f"gated attention, rows {place} T={T} past={past}", flush=True)
+    x, q_proj, k_proj, qw, kw = _case(800 + T, T, hq, hkv, d, past)
+    ref, out, caches, _ = _run_both(gpu, x, q_proj, k_proj, qw, kw, past, 64)
+    assert torch.equal(ref, out)
+    f32 = lambda a: torch.from_numpy(a).to(gpu)
+    qp, kp, vn = u16_to_torch(q_proj, gpu), u16_to_torch(k_proj, gpu), u16_to_torch(x.v_new, gpu)
+    kc, vc = u16_to_torch(x.k_cache, gpu), u16_to_torch(x.v_cache, gpu)
+    kc[past:] = 0
+    vc[past:] = 0
+    out = torch.zeros(T, hq, d, dtype=torch.float16, device=gpu)
+    if place == "unaligned":
+        room = torch.empty(2, T * hkv * d + 8, dtype=torch.float16, device=gpu)
+        k, v = (room[i, 1:1 + T * hkv * d].view(T, hkv, d) for i in range(2))
+        k.copy_(kp)
+        v.copy_(vn)
+    else:
+        k = vc[past:past + T] if place == "keys_in_values" else \
+            out.view(-1)[:T * hkv * d].view(T, hkv, d)
+        k.copy_(kp)
+        v = vn
+    got = ops.gated_attention(qp, k, v, f32(qw), f32(kw), kc, vc, past, 64, EPS, THETA, out=out)
+    torch.cuda.synchronize()
+    assert torch.equal(caches[0], kc) and torch.equal(caches[1], vc)
+    assert torch.equal(ref, got)
+
+
 @pytest.mark.parametrize("T,past,hq,hkv", [(1, 4096, 16, 4), (40, 24, 16, 4), (100, 37, 64, 16)])
 def test_fused_block_against_the_oracle(gpu, T, past, hq, hkv):
     d, rot = 256, 64

@@ -1,0 +1,43 @@
+"""The library's host code without a GPU: which kernels a call launches.
+
+tests/host_runtime.cpp links the library and defines the HIP runtime calls it
+makes; its commands run entry points over host memory and print the launches.
+"""
+import os
+import subprocess
+
+import pytest
+
+from llminfer_amd import _lib
+from tests.conftest import ROOT
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    """run(command, *args, env={}) -> [(what, [word, ...]), ...]"""
+    exe = tmp_path_factory.mktemp("host") / "host_runtime"
+    lib = _lib.LIB_PATH
+    subprocess.run(["g++", "-std=c++17", "-O1", "-rdynamic", "-D__HIP_PLATFORM_AMD__",
+                    f"-I{ROOT}/include", "-I/opt/rocm/include", f"{ROOT}/tests/host_runtime.cpp",
+                    str(lib), f"-Wl,-rpath,{lib.parent}", "-Wl,-rpath-link,/opt/rocm/lib",
+                    "-o", str(exe)], check=True)
+
+    def run(*args, env=None):
+        out = subprocess.run([str(exe), *map(str, args)], check=True, capture_output=True,
+                             text=True, timeout=60, env={**os.environ, **(env or {})}).stdout
+        return [(line.split()[0], line.split()[1:]) for line in out.splitlines()]
+    return run
+
+
+@pytest.mark.parametrize("place,joint", [
+    ("apart", True), ("keys_in_values", False), ("values_in_keys", False),
+    ("keys_in_output", False), ("keys_unaligned", False)])
+def test_gated_prefill_rows_share_a_launch_only_where_order_does_not_matter(host, place, joint):
+    got = dict(host("gated", 40, 24, 16, 4, 256, 64, place))
+    assert got["status"] == ["0"]
+    rows = got["launches"][:-1]
+    if joint:
+        assert rows == ["attention_rows"]
+    else:  # the keys, the values, the queries
+        keys = "norm_rope_rows" if place == "keys_unaligned" else "norm_rope_tile"
+        assert rows == [keys, "kv_append_vec", "norm_rope_tile"]
