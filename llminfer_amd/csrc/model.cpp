@@ -441,18 +441,21 @@ size_t state_bytes(const llmi_graph_state &s) {
   return n;
 }
 
-// fp16 to fp32, exact: the exponent is rebiased by a product with 2^112, which
-// also normalises subnormals; infinities and NaNs keep their fraction. No
-// branches, so the logits' loop runs on vector registers.
+// fp16 to fp32, exact in any floating-point mode: the exponent is rebiased as a
+// whole number, and a subnormal's fraction, as one too, is scaled by 2^-24 (no
+// fp32 subnormal, which denormals-are-zero would lose). Infinities and NaNs keep
+// their fraction. Selects and no branches, so the logits' loop runs on vector
+// registers.
 float half_to_float(uint16_t h) {
   const uint32_t sign = (uint32_t)(h & 0x8000u) << 16, low = (uint32_t)(h & 0x7FFFu) << 13;
-  float x;
-  std::memcpy(&x, &low, 4);
-  x *= 0x1p112f;
-  uint32_t bits;
-  std::memcpy(&bits, &x, 4);
+  const float small = (float)(int)(h & 0x3FFu) * 0x1p-24f;
+  uint32_t fraction;
+  std::memcpy(&fraction, &small, 4);
+  uint32_t bits = low + (112u << 23);
   bits = (h & 0x7C00u) == 0x7C00u ? low | 0x7F800000u : bits;
+  bits = (h & 0x7C00u) == 0 ? fraction : bits;
   bits |= sign;
+  float x;
   std::memcpy(&x, &bits, 4);
   return x;
 }

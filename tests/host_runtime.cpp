@@ -7,6 +7,7 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -180,11 +181,76 @@ int gated(char **a) {
   return 0;
 }
 
+// A two-layer model whose kernels do not run: its logits are what the device
+// buffer held, the 65,536 fp16 values.
+struct Model {
+  std::vector<uint8_t> kinds{0, 1}; // DeltaNet, GQA
+  llmi_qwen35_config c{};
+  std::vector<llmi_named_weight> weights;
+  llmi_qwen35_graph *graph = nullptr;
+  llmi_hip_model *session = nullptr;
+
+  explicit Model(uint64_t capacity) {
+    c.hidden = 512, c.intermediate = 1024, c.vocabulary = 65536, c.max_positions = 1 << 16;
+    c.head_dim = 256, c.q_heads = 4, c.kv_heads = 2, c.rotary_width = 64;
+    c.key_heads = 2, c.value_heads = 4, c.key_dim = 128, c.value_dim = 128, c.conv_kernel = 4;
+    c.epsilon = 1e-6, c.theta = 1e7, c.w8 = 1;
+    c.layer_count = (uint32_t)kinds.size(), c.layer_kinds = kinds.data();
+    static unsigned char data[16];
+    if (llmi_qwen35_build(&c, 1, 0, capacity, LLMI_LOGITS_ALL, &graph) != LLMI_HIP_OK)
+      abort();
+    for (size_t i = 0; i < llmi_qwen35_graph_tensor_count(graph); ++i)
+      weights.push_back({llmi_qwen35_graph_tensor(graph, i), data, (const uint16_t *)data});
+    if (llmi_hip_model_open(&c, weights.data(), weights.size(), capacity, nullptr, &session)) {
+      fprintf(stderr, "%s\n", llmi_hip_last_error());
+      abort();
+    }
+  }
+  ~Model() {
+    llmi_hip_model_close(session);
+    llmi_qwen35_graph_destroy(graph);
+  }
+};
+
+double half_value(unsigned h) {
+  const int e = h >> 10 & 0x1F, f = h & 0x3FF;
+  const double m = e == 0x1F ? (f ? NAN : INFINITY)
+                   : e       ? ldexp(1024 + f, e - 25)
+                             : ldexp(f, -24);
+  return h & 0x8000 ? -m : m;
+}
+
+// logits MXCSR: the wrong ones of a step's logits, with the thread's
+// floating-point control bits set.
+int logits(char **a) {
+  Model m(8);
+  std::vector<float> out(65536);
+  const uint32_t token = 1;
+  _mm_setcsr(_mm_getcsr() | (unsigned)strtoul(a[0], nullptr, 0));
+  printf("status %d\n", llmi_hip_model_step(m.session, &token, 1, LLMI_LOGITS_LAST, out.data(),
+                                            out.size(), nullptr));
+  size_t wrong = 0;
+  for (unsigned h = 0; h < 65536; ++h) {
+    const double want = half_value(h);
+    const float exact = (float)want; // (no fp16 value is an fp32 subnormal)
+    uint32_t bits, expected;
+    memcpy(&bits, &out[h], 4);
+    memcpy(&expected, &exact, 4);
+    if (std::isnan(want))
+      expected = (h & 0x8000u) << 16 | 0x7F800000u | (h & 0x3FFu) << 13;
+    wrong += bits != expected;
+  }
+  printf("wrong %zu\n", wrong);
+  return 0;
+}
+
 } // namespace
 
 int main(int argc, char **argv) {
   const std::string command = argc > 1 ? argv[1] : "";
   if (command == "gated" && argc == 9)
     return gated(argv + 2);
+  if (command == "logits" && argc == 3)
+    return logits(argv + 2);
   return 2;
 }

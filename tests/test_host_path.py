@@ -41,3 +41,11 @@ def test_gated_prefill_rows_share_a_launch_only_where_order_does_not_matter(host
     else:  # the keys, the values, the queries
         keys = "norm_rope_rows" if place == "keys_unaligned" else "norm_rope_tile"
         assert rows == [keys, "kv_append_vec", "norm_rope_tile"]
+
+
+@pytest.mark.parametrize("mxcsr", [0, 0x8040])  # the default, and FTZ + DAZ
+def test_logits_are_exact_in_any_float_mode(host, mxcsr):
+    """Every fp16 value as a logit, read by a thread that flushes denormals
+    (torch.set_flush_denormal(True) sets the same two bits)."""
+    got = dict(host("logits", mxcsr))
+    assert got["status"] == ["0"] and got["wrong"] == ["0"]
