@@ -156,6 +156,9 @@ __global__ __launch_bounds__(256) void causal_conv_k4(
   }
 }
 
+// A half of a word that was stored whole: the two stores must stay in order.
+typedef uint16_t __attribute__((may_alias)) word_half_t;
+
 // The 4-tap case of several tokens, two channels a lane and eight tokens: as
 // many outputs a lane in half the loads and stores. The estimates of the SiLU
 // first, then the exact values over those that did not settle: about one in
@@ -223,7 +226,7 @@ __global__ __launch_bounds__(256, 8) void causal_conv_k4_pairs(
       hk = k == i ? h[i] : hk;
     const unsigned t = t0 + k / 2;
     if (t < T)
-      reinterpret_cast<uint16_t *>(out)[(t * pairs + c) * 2 + (k & 1)] =
+      reinterpret_cast<word_half_t *>(out)[(t * pairs + c) * 2 + (k & 1)] =
           f2h(mul32(hk, logistic_exact(hk)));
   }
   if (t0 == 0) {
