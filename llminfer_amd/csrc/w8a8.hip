@@ -445,7 +445,8 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemv_split_kernel(
 // A step covers 8 groups: 256 bytes of each of the tile's 32 activation and 32
 // weight rows go HBM -> LDS with buffer loads that write LDS directly, double
 // buffered; the scales come through registers, requested a step before they
-// are staged. One barrier a step, and no wait there for the scales.
+// are staged. One barrier a step, behind a wait for everything but the last
+// request of scales.
 // Measured (weights rotating past the MALL; 512 rows of 2560 -> 9216, 512 of
 // 9216 -> 2560, 128 of 2560 -> 9216, 13 of 9216 -> 2560):
 //   through registers and a padded layout      74.4, 73.4, 24.5, 58.1 us
@@ -558,23 +559,27 @@ __global__ __launch_bounds__(kGemmThreads, 4) void gemm_kernel(
       acc[4 * q + 3] = add_term(acc[4 * q + 3], dots[4 * q + 3], a4[q].w, wsv);
     }
   };
-  // A step: the next one's loads go out, this one's arithmetic runs, the next
-  // one's scale (requested a step ago) is staged and the one after requested.
-  // The wait before the barrier is for everything but that last request.
+  // A step: the next one's loads go out, this one's arithmetic runs, and once
+  // this wave's loads have landed (the next step's rows and its scale, requested
+  // a step ago) that scale is staged and the one after requested, which alone
+  // is in flight at the barrier: it ends in a register.
+  auto landed = [] { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
   auto run = [&](unsigned step, const unsigned char *st, unsigned char *next) {
     if (step + 1 < nsteps)
       load(next);
     if (step * kSpan + wave < p.groups)
       compute(st, sc[step % 2]);
+    landed();
     stage_scale(sc[(step + 1) % 2]);
     load_scale(step + 2);
-    asm volatile("s_waitcnt vmcnt(1) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    lds_sync();
   };
   load(s0);
   load_scale(0);
+  landed();
   stage_scale(sc[0]);
   load_scale(1);
-  asm volatile("s_waitcnt vmcnt(1) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  lds_sync();
   for (unsigned step = 0; step < nsteps; step += 2) {
     run(step, s0, s1);
     if (step + 1 < nsteps)
