@@ -643,8 +643,9 @@ LLMI_HIP_API int llmi_hip_workspace_init(void *workspace, size_t bytes, void *st
 
 /* Plan-record support (MetalSession.h:11-16, tools/run/Main.cpp:244-255):
  * the number of kernel launches an op lowers to and the name of launch
- * `index`. `params` points to the op's parameter struct. NULL / 0 on a
- * parameter set the backend rejects. */
+ * `index`, for 16-byte aligned buffers apart from each other and the workspace
+ * that the op's query asks for. `params` points to the op's parameter struct.
+ * NULL / 0 on a parameter set the backend rejects. */
 LLMI_HIP_API unsigned llmi_hip_dispatch_count(int op, const void *params);
 LLMI_HIP_API const char *llmi_hip_kernel_name(int op, const void *params, unsigned index);
 

@@ -984,6 +984,12 @@ int llmi_hip_workspace_init(void *workspace, size_t bytes, void *stream) {
                   "workspace_init");
 }
 
+// Whether a supported CausalGqa is a prefill that divides its keys.
+static bool prefill_merges(const GqaParams &p) {
+  return select_gqa(p) == GqaKernel::Prefill &&
+         prefill_split({p.tokens, p.queryHeads, p.kvHeads, p.headDim, p.past});
+}
+
 unsigned llmi_hip_dispatch_count(int op, const void *params) {
   if (!params)
     return 0;
@@ -996,7 +1002,7 @@ unsigned llmi_hip_dispatch_count(int op, const void *params) {
       return 0;
     if (select_gqa(p) == GqaKernel::Decode)
       return decode_launches({p.tokens, p.queryHeads, p.kvHeads, p.headDim, p.past});
-    return 1; // (the merge of a prefill that divides its keys belongs to it)
+    return prefill_merges(p) ? 2 : 1;
   }
   case LLMI_HIP_OP_KV_APPEND_CAUSAL_GQA: {
     const GqaParams &p = *static_cast<const GqaParams *>(params);
@@ -1008,7 +1014,7 @@ unsigned llmi_hip_dispatch_count(int op, const void *params) {
     case GqaKernel::None:
       return 0;
     default:
-      return 2;
+      return prefill_merges(p) ? 3 : 2;
     }
   }
   case LLMI_HIP_OP_DELTA_UPDATE: {
@@ -1091,7 +1097,9 @@ unsigned llmi_hip_dispatch_count(int op, const void *params) {
     GqaShape s{p.tokens, p.queryHeads, p.kvHeads, p.headDim, p.past};
     if (decode_gated_supported(s, 16))
       return decode_launches(s);
-    return p.tokens > 1 && prefill_gated_supported(s, 16) ? 3 : 0;
+    if (p.tokens < 2 || !prefill_gated_supported(s, 16))
+      return 0;
+    return prefill_split(s) ? 3 : 2;
   }
   }
   return 0;
@@ -1106,14 +1114,14 @@ const char *llmi_hip_kernel_name(int op, const void *params, unsigned index) {
   case LLMI_HIP_OP_KV_APPEND_CAUSAL_GQA:
     if (select_gqa(*static_cast<const GqaParams *>(params)) != GqaKernel::Decode)
       return index == 0 ? "kvAppend"
-                        : llmi_hip_kernel_name(LLMI_HIP_OP_CAUSAL_GQA, params, 0);
+                        : llmi_hip_kernel_name(LLMI_HIP_OP_CAUSAL_GQA, params, index - 1);
     return llmi_hip_kernel_name(LLMI_HIP_OP_CAUSAL_GQA, params, index);
   case LLMI_HIP_OP_CAUSAL_GQA:
     switch (select_gqa(*static_cast<const GqaParams *>(params))) {
     case GqaKernel::Decode:
       return index == 0 ? "gqaDecodeSplitK" : "gqaDecodeMerge";
     case GqaKernel::Prefill:
-      return "gqaPrefillMfma";
+      return index == 0 ? "gqaPrefillMfma" : "gqaPrefillMerge";
     case GqaKernel::Generic:
       return "gqaGeneric";
     case GqaKernel::None:
@@ -1193,7 +1201,11 @@ const char *llmi_hip_kernel_name(int op, const void *params, unsigned index) {
   case LLMI_HIP_OP_GATED_ATTENTION:
     if (static_cast<const GqaParams *>(params)->tokens == 1)
       return index == 0 ? "gqaDecodeGated" : "gqaDecodeMergeGated";
-    return index == 0 ? "normRopeTile" : index == 1 ? "cacheAppend" : "gqaPrefillGated";
+    if (index == 0) // (for 16-byte aligned rows apart from the outputs)
+      return "attentionRows";
+    if (llmi_hip_dispatch_count(op, params) == 2)
+      return "gqaPrefillGated";
+    return index == 1 ? "gqaPrefillMfma" : "gqaPrefillMergeGated";
   }
   return nullptr;
 }

@@ -284,7 +284,7 @@ int llmi_hip_session_step(llmi_hip_session *s, unsigned tokens, const float *dq,
   // Plan records, in graph order: DeltaUpdate (op 0), KvAppend (op 1),
   // CausalGqa (op 2). KvAppend and CausalGqa run through the fused entry
   // point: one decode launch that also appends (recorded under op 1 and
-  // again under op 2), or append then prefill.
+  // again under op 2), or append then prefill (and its merge).
   size_t n = 0;
   for (unsigned i = 0, m = llmi_hip_dispatch_count(LLMI_HIP_OP_DELTA_UPDATE, &dp); i < m; ++i)
     record(records, cap, n, 0, llmi_hip_kernel_name(LLMI_HIP_OP_DELTA_UPDATE, &dp, i));
@@ -300,8 +300,9 @@ int llmi_hip_session_step(llmi_hip_session *s, unsigned tokens, const float *dq,
   } else {
     record(records, cap, n, 1,
            llmi_hip_kernel_name(LLMI_HIP_OP_KV_APPEND_CAUSAL_GQA, &gp, 0));
-    record(records, cap, n, 2,
-           llmi_hip_kernel_name(LLMI_HIP_OP_KV_APPEND_CAUSAL_GQA, &gp, 1));
+    for (unsigned i = 1; i < pairLaunches; ++i)
+      record(records, cap, n, 2,
+             llmi_hip_kernel_name(LLMI_HIP_OP_KV_APPEND_CAUSAL_GQA, &gp, i));
   }
   if (count)
     *count = n;

@@ -212,6 +212,31 @@ struct Model {
   }
 };
 
+// gqa T past q_heads kv_heads head_dim fused: a CausalGqa, with its KvAppend
+// if fused.
+int gqa(char **a) {
+  const GqaParams p{(unsigned)atoi(a[0]), (unsigned)atoi(a[2]), (unsigned)atoi(a[3]),
+                    (unsigned)atoi(a[4]), (unsigned)atoi(a[1])};
+  const size_t q = (size_t)p.tokens * p.queryHeads * p.headDim,
+               rows = (size_t)(p.past + p.tokens) * p.kvHeads * p.headDim,
+               bytes = llmi_hip_gqa_workspace_bytes(p);
+  void *m[7];
+  const size_t n[7] = {2 * q, 2 * q, 2 * rows, 2 * rows, 2 * rows, 2 * rows, bytes};
+  for (int i = 0; i < 7; ++i)
+    if (hipMalloc(&m[i], n[i]) != hipSuccess)
+      return 1;
+  auto u16 = [&](int i) { return static_cast<uint16_t *>(m[i]); };
+  const bool fused = atoi(a[5]);
+  launches.clear();
+  printf("status %d\n",
+         fused ? llmi_hip_kv_append_causal_gqa(u16(0), u16(2), u16(3), u16(4), u16(5), u16(1), p,
+                                               m[6], bytes, nullptr)
+               : llmi_hip_causal_gqa(u16(0), u16(4), u16(5), u16(1), p, m[6], bytes, nullptr));
+  flush_launches("launches");
+  names(fused ? LLMI_HIP_OP_KV_APPEND_CAUSAL_GQA : LLMI_HIP_OP_CAUSAL_GQA, p);
+  return 0;
+}
+
 double half_value(unsigned h) {
   const int e = h >> 10 & 0x1F, f = h & 0x3FF;
   const double m = e == 0x1F ? (f ? NAN : INFINITY)
@@ -250,6 +275,8 @@ int main(int argc, char **argv) {
   const std::string command = argc > 1 ? argv[1] : "";
   if (command == "gated" && argc == 9)
     return gated(argv + 2);
+  if (command == "gqa" && argc == 8)
+    return gqa(argv + 2);
   if (command == "logits" && argc == 3)
     return logits(argv + 2);
   return 2;

@@ -8,8 +8,8 @@ the key cache, cacheAppend of the values, the attention, and the sigmoid gate
 same sequence through this backend's standalone launches -- each bit-exact
 with the oracle in the row-op tests -- must give exactly the fused call's
 output and cache bits, at the decode (one launch + merge) and prefill
-(K normRope + append, then the MFMA prefill with q normRope in its load and
-the gate in its store) shapes. Two cases are also checked end to end against
+(the rows' launch, then the MFMA prefill with the gate in its store or its
+merge) shapes. Two cases are also checked end to end against
 the oracle: oracle normRope and sigmoidMul around the double-precision
 attention, within the north-star 2e-3. The activated form
 (llmi_hip_gated_attention_activated: the gate half already holds
@@ -82,13 +82,13 @@ def test_fused_block_equals_the_unfused_ops(gpu, T, past, shape, rot):
     if T == 1:
         assert names[0] == "gqaDecodeGated"
     else:
-        assert names == ["normRopeTile", "cacheAppend", "gqaPrefillGated"]
+        assert names == ["attentionRows", "gqaPrefillGated"]
 
 
 @pytest.mark.parametrize("T,past,shape,rot", [
     (3, 515, (16, 4, 256), 64), (61, 1500, (16, 4, 256), 128), (40, 700, (16, 4, 128), 32)])
 def test_divided_block_equals_the_unfused_ops(gpu, T, past, shape, rot):
-    """A prefill that divides its keys: q normalised into the workspace, the
+    """A prefill that divides its keys: q normalised into the output, the
     merge gates."""
     hq, hkv, d = shape
     print(f"divided gated attention T={T} past={past} shape={shape} rot={rot}", flush=True)
@@ -96,7 +96,10 @@ def test_divided_block_equals_the_unfused_ops(gpu, T, past, shape, rot):
     ref, out, caches_ref, caches = _run_both(gpu, x, q_proj, k_proj, qw, kw, past, rot)
     assert torch.equal(caches_ref[0], caches[0]) and torch.equal(caches_ref[1], caches[1])
     assert torch.equal(ref, out), "output differs from the unfused ops"
-    assert _lib.load().llmi_hip_gqa_workspace_bytes(_lib.GqaParams(T, hq, hkv, d, past)) > 0
+    p = _lib.GqaParams(T, hq, hkv, d, past)
+    assert _lib.load().llmi_hip_gqa_workspace_bytes(p) > 0
+    assert ops.kernel_names(_lib.OP_GATED_ATTENTION, p) == \
+        ["attentionRows", "gqaPrefillMfma", "gqaPrefillMergeGated"]
 
 
 @pytest.mark.parametrize("place", ["keys_in_values", "keys_in_output", "unaligned"])

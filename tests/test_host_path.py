@@ -49,3 +49,29 @@ def test_logits_are_exact_in_any_float_mode(host, mxcsr):
     (torch.set_flush_denormal(True) sets the same two bits)."""
     got = dict(host("logits", mxcsr))
     assert got["status"] == ["0"] and got["wrong"] == ["0"]
+
+
+# The kernel of each record's name.
+KERNELS = {"kvAppend": "kv_append_vec", "gqaDecodeSplitK": "gqa_decode_split_kernel",
+           "gqaDecodeMerge": "gqa_decode_merge_kernel", "gqaPrefillMfma": "gqa_prefill",
+           "gqaPrefillGated": "gqa_prefill", "gqaPrefillMerge": "gqa_prefill_merge_kernel",
+           "gqaPrefillMergeGated": "gqa_prefill_merge_kernel", "gqaGeneric": "gqa_generic",
+           "attentionRows": "attention_rows"}
+
+
+@pytest.mark.parametrize("T,past,hq,hkv,d", [
+    (2, 0, 16, 4, 256), (61, 511, 16, 4, 256), (61, 512, 16, 4, 256), (2, 4000, 16, 4, 128),
+    (40, 700, 8, 1, 256), (512, 2000, 8, 8, 128), (2048, 2048, 16, 4, 256), (3, 600, 4, 2, 64)])
+@pytest.mark.parametrize("call", ["gqa", "append", "gated"])
+def test_records_name_what_is_launched(host, call, T, past, hq, hkv, d):
+    if call == "gated":
+        got = dict(host("gated", T, past, hq, hkv, d, 32, "apart"))
+        if d < 128:
+            assert got["status"] != ["0"] and got["names"] == []
+            return
+    else:
+        got = dict(host("gqa", T, past, hq, hkv, d, int(call == "append")))
+    assert got["status"] == ["0"]
+    assert len(got["names"]) == len(got["launches"])
+    for name, kernel in zip(got["names"], got["launches"]):
+        assert kernel.startswith(KERNELS[name])
