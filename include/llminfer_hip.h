@@ -727,8 +727,9 @@ LLMI_HIP_API int llmi_hip_session_check(const llmi_hip_session_config *config,
  * nonzero before any launch. If `records` is non-NULL, up to `cap` plan
  * records are written and *count receives the total; for T == 1 KvAppend
  * runs inside the attention launch, which is recorded under op 1 and again
- * under op 2. The step waits for the GPU once at the end (one host sync per
- * step, MetalContext.mm:141-151). */
+ * under op 2; a prefill whose divided keys' partials find no device memory
+ * runs undivided, and records no merge. The step waits for the GPU once at the
+ * end (one host sync per step, MetalContext.mm:141-151). */
 LLMI_HIP_API int llmi_hip_session_step(llmi_hip_session *s, unsigned tokens,
                           const float *dq, const float *dk, const uint16_t *dv,
                           const float *beta, const float *decay,

@@ -20,6 +20,7 @@
 #include "kernels.hpp"
 
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <new>
 #include <string.h>
 
@@ -110,9 +111,11 @@ int ensure_workspace(llmi_hip_session *s, size_t need) {
   if (need <= s->wsBytes)
     return LLMI_HIP_OK;
   void *ws = nullptr;
-  if (hipMalloc(&ws, need) != hipSuccess)
+  if (hipMalloc(&ws, need) != hipSuccess) {
+    (void)hipGetLastError(); // the step may run without it
     return fail(LLMI_HIP_WORKSPACE, "session: cannot allocate a %zu-byte workspace",
                 need);
+  }
   if (s->ws)
     (void)hipFree(s->ws);
   s->ws = ws;
@@ -274,12 +277,16 @@ int llmi_hip_session_step(llmi_hip_session *s, unsigned tokens, const float *dq,
   const llmi_hip_session_config &c = s->cfg;
   GraphDeltaParams dp{tokens, c.keyHeads, c.keyDim, c.valueHeads, c.valueDim};
   GqaParams gp{tokens, c.queryHeads, c.kvHeads, c.headDim, s->past};
-  size_t need = llmi_hip_gqa_workspace_bytes(gp);
-  size_t needDelta = llmi_hip_delta_workspace_bytes(dp);
-  if (needDelta > need)
-    need = needDelta;
-  if (int st = ensure_workspace(s, need))
-    return st;
+  // The two ops use the workspace in turn. A prefill that finds no room for
+  // the partials of its divided keys runs undivided.
+  const size_t needGqa = llmi_hip_gqa_workspace_bytes(gp);
+  const size_t needDelta = llmi_hip_delta_workspace_bytes(dp);
+  const bool prefill = select_gqa(gp) == GqaKernel::Prefill;
+  int room = ensure_workspace(s, std::max(needGqa, needDelta));
+  if (room != LLMI_HIP_OK && prefill)
+    room = ensure_workspace(s, needDelta);
+  if (room != LLMI_HIP_OK)
+    return room;
 
   // Plan records, in graph order: DeltaUpdate (op 0), KvAppend (op 1),
   // CausalGqa (op 2). KvAppend and CausalGqa run through the fused entry
@@ -300,7 +307,8 @@ int llmi_hip_session_step(llmi_hip_session *s, unsigned tokens, const float *dq,
   } else {
     record(records, cap, n, 1,
            llmi_hip_kernel_name(LLMI_HIP_OP_KV_APPEND_CAUSAL_GQA, &gp, 0));
-    for (unsigned i = 1; i < pairLaunches; ++i)
+    const unsigned ran = prefill && s->wsBytes < needGqa ? 2 : pairLaunches;
+    for (unsigned i = 1; i < ran; ++i)
       record(records, cap, n, 2,
              llmi_hip_kernel_name(LLMI_HIP_OP_KV_APPEND_CAUSAL_GQA, &gp, i));
   }

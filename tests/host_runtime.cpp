@@ -237,6 +237,34 @@ int gqa(char **a) {
   return 0;
 }
 
+// session past tokens limit: a step of the layer-pair session whose new
+// allocations may take up to `limit` bytes each.
+int session(char **a) {
+  const unsigned past = atoi(a[0]), tokens = atoi(a[1]);
+  const llmi_hip_session_config c{past + tokens, 16, 4, 256, 16, 128, 32, 128};
+  llmi_hip_session *s = nullptr;
+  if (llmi_hip_session_open(&c, nullptr, &s) || llmi_hip_session_restore(s, past))
+    return 1;
+  void *x; // (read by nothing: the kernels do not run)
+  if (hipMalloc(&x, 1 << 20) != hipSuccess)
+    return 1;
+  auto *f = static_cast<float *>(x);
+  auto *u = static_cast<uint16_t *>(x);
+  llmi_hip_dispatch records[16];
+  size_t count = 0;
+  largest = strtoull(a[2], nullptr, 0);
+  launches.clear();
+  printf("status %d\n", llmi_hip_session_step(s, tokens, f, f, u, f, f, u, u, u, u, u, records, 16,
+                                               &count));
+  flush_launches("launches");
+  printf("names");
+  for (size_t i = 0; i < count; ++i)
+    printf(" %s", records[i].kernel);
+  printf("\npast %u\n", llmi_hip_session_past(s));
+  llmi_hip_session_close(s);
+  return 0;
+}
+
 double half_value(unsigned h) {
   const int e = h >> 10 & 0x1F, f = h & 0x3FF;
   const double m = e == 0x1F ? (f ? NAN : INFINITY)
@@ -277,6 +305,8 @@ int main(int argc, char **argv) {
     return gated(argv + 2);
   if (command == "gqa" && argc == 8)
     return gqa(argv + 2);
+  if (command == "session" && argc == 5)
+    return session(argv + 2);
   if (command == "logits" && argc == 3)
     return logits(argv + 2);
   return 2;

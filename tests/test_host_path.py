@@ -75,3 +75,24 @@ def test_records_name_what_is_launched(host, call, T, past, hq, hkv, d):
     assert len(got["names"]) == len(got["launches"])
     for name, kernel in zip(got["names"], got["launches"]):
         assert kernel.startswith(KERNELS[name])
+
+
+NO_LIMIT = 2 ** 63
+
+
+@pytest.mark.parametrize("tokens,limit,divided", [
+    (61, NO_LIMIT, True), (61, 8 << 20, False), (1, NO_LIMIT, None)])
+def test_session_step_runs_undivided_where_the_partials_find_no_room(host, tokens, limit, divided):
+    got = dict(host("session", 16411, tokens, limit))
+    assert got["status"] == ["0"] and got["past"] == [str(16411 + tokens)]
+    if divided is not None:
+        merges = [n for n in got["launches"] if "prefill_merge" in n]
+        assert len(merges) == divided
+        assert got["names"].count("gqaPrefillMerge") == divided
+        assert got["names"].count("gqaPrefillMfma") == 1
+
+
+def test_session_step_without_a_decode_workspace_is_refused(host):
+    got = dict(host("session", 16411, 1, 1 << 16))
+    assert got["status"] == [str(_lib.WORKSPACE)] and got["launches"] == []
+    assert got["past"] == ["16411"]
