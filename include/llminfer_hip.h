@@ -837,7 +837,11 @@ LLMI_HIP_API int llmi_hip_plan_lower(const llmi_graph *graph, const llmi_weight 
                                      size_t weight_count, llmi_hip_plan **out);
 LLMI_HIP_API void llmi_hip_plan_destroy(llmi_hip_plan *plan);
 
-/* Bytes of the scratch arena llmi_hip_plan_execute needs (256-aligned). */
+/* Bytes of the scratch arena of llmi_hip_plan_execute (256-aligned). Where the
+ * step's prefills divide their keys, their partials are its last
+ * llmi_hip_gqa_workspace_bytes bytes (rounded up to 256): an arena without
+ * these is taken too, and the prefills then run undivided, without the merges
+ * that the plan's records name. */
 LLMI_HIP_API size_t llmi_hip_plan_scratch_bytes(const llmi_hip_plan *plan);
 
 /* The logits output: rows and elements (0 when the graph has no output). */

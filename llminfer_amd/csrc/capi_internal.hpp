@@ -29,6 +29,9 @@ int run_gqa(const uint16_t *q, const uint16_t *k_new, const uint16_t *v_new,
             const GqaParams &p, void *workspace, size_t workspace_bytes,
             void *stream);
 
+// Bytes of a plan's scratch arena that it runs without, its prefills undivided.
+size_t plan_partial_bytes(const llmi_hip_plan *plan);
+
 // Launch count and names of the chunked DeltaNet path (delta_chunked.hip).
 unsigned delta_chunked_dispatches();
 const char *delta_chunked_kernel_name(unsigned index);

@@ -539,13 +539,25 @@ int grow(void **buf, size_t &have, size_t need, hipStream_t stream, const char *
     return LLMI_HIP_OK;
   (void)hipStreamSynchronize(stream);
   void *p = nullptr;
-  if (hipMalloc(&p, need) != hipSuccess)
+  if (hipMalloc(&p, need) != hipSuccess) {
+    (void)hipGetLastError(); // the step may run without it
     return fail(LLMI_HIP_WORKSPACE, "model: cannot allocate %zu bytes of %s", need, what);
+  }
   if (*buf)
     (void)hipFree(*buf);
   *buf = p;
   have = need;
   return LLMI_HIP_OK;
+}
+
+// The scratch arena of a plan: the whole, or where there is no room for it the
+// part without its divided prefills' partials.
+int grow_scratch(llmi_hip_model *s, const llmi_hip_plan *plan) {
+  const size_t whole = llmi_hip_plan_scratch_bytes(plan), partials = plan_partial_bytes(plan);
+  const int st = grow(&s->scratch, s->scratchBytes, whole, s->stream, "scratch");
+  return st == LLMI_HIP_OK || !partials
+             ? st
+             : grow(&s->scratch, s->scratchBytes, whole - partials, s->stream, "scratch");
 }
 
 // The plan of a step graph over the model's weights.
@@ -769,8 +781,7 @@ int llmi_hip_model_step(llmi_hip_model *s, const uint32_t *ids, size_t count, in
   if (elements && (!logits || logits_capacity < elements))
     return fail(LLMI_HIP_INVALID_ARGUMENT, "model: logits need %llu floats",
                 (unsigned long long)elements);
-  if (int st = grow(&s->scratch, s->scratchBytes, llmi_hip_plan_scratch_bytes(plan.p),
-                    s->stream, "scratch"))
+  if (int st = grow_scratch(s, plan.p))
     return st;
   if (int st = grow(reinterpret_cast<void **>(&s->logits), s->logitBytes, elements * 2,
                     s->stream, "logits"))
@@ -812,11 +823,19 @@ int llmi_hip_model_step(llmi_hip_model *s, const uint32_t *ids, size_t count, in
   }
   read_logits(half, logits, elements);
   s->past += count;
-  const size_t n = llmi_hip_plan_dispatches(plan.p, nullptr, 0);
-  s->records.resize(n);
-  llmi_hip_plan_dispatches(plan.p, s->records.data(), n);
+  size_t scratch = llmi_hip_plan_scratch_bytes(plan.p);
+  s->records.resize(llmi_hip_plan_dispatches(plan.p, nullptr, 0));
+  llmi_hip_plan_dispatches(plan.p, s->records.data(), s->records.size());
+  if (s->scratchBytes < scratch) { // its prefills ran undivided, without their merges
+    scratch -= plan_partial_bytes(plan.p);
+    s->records.erase(std::remove_if(s->records.begin(), s->records.end(),
+                                    [](const llmi_hip_dispatch &d) {
+                                      return !std::strcmp(d.kernel, "gqaPrefillMerge");
+                                    }),
+                     s->records.end());
+  }
   if (result)
-    *result = llmi_hip_model_step_result{s->past, rows, llmi_hip_plan_scratch_bytes(plan.p), n};
+    *result = llmi_hip_model_step_result{s->past, rows, scratch, s->records.size()};
   return LLMI_HIP_OK;
 }
 
@@ -874,8 +893,7 @@ int llmi_hip_model_run(llmi_hip_model *s, const llmi_hip_plan *plan, const uint3
     return fail(LLMI_HIP_INVALID_ARGUMENT, "model: null argument");
   if (s->invalid)
     return fail(LLMI_HIP_INVALID_ARGUMENT, "Session is invalid after a failed GPU step");
-  if (int st = grow(&s->scratch, s->scratchBytes, llmi_hip_plan_scratch_bytes(plan), s->stream,
-                    "scratch"))
+  if (int st = grow_scratch(s, plan))
     return st;
   return llmi_hip_plan_execute(plan, s->scratch, s->scratchBytes, s->states.data(),
                                s->states.size(), ids, logits, s->flag, s->stream);

@@ -28,7 +28,11 @@ namespace {
 
 constexpr uint64_t kAlign = 256;
 
-enum class Space : uint8_t { None, Scratch, Weight, Scale, State, Input, Output, Invalid };
+// Partials: the tail of the scratch arena, for prefills that divide their keys
+// (null, and so undivided, where the caller's arena ends before it).
+enum class Space : uint8_t {
+  None, Scratch, Partials, Weight, Scale, State, Input, Output, Invalid
+};
 
 // A device address resolved at run time: the base of `space` (entry `index`
 // of the weight or state table) plus `offset` bytes.
@@ -133,7 +137,7 @@ struct llmi_hip_plan {
   std::vector<llmi::Dispatch> dispatches;
   std::vector<llmi_hip_dispatch> records;
   std::vector<llmi_weight> weights;
-  uint64_t scratchBytes = 0;
+  uint64_t scratchBytes = 0, partialBytes = 0; // the arena, and its tail's share of it
   uint64_t logitRows = 0, logitElements = 0;
   uint64_t invalidOffset = 0;
   size_t stateCount = 0;
@@ -1346,8 +1350,12 @@ int Lowering::lower(size_t i) {
       d.kernels.push_back(llmi_hip_kernel_name(LLMI_HIP_OP_CAUSAL_GQA, &p, k));
     d.buf[0] = r[0], d.buf[1] = state(o.keys), d.buf[2] = state(o.values), d.buf[3] = r[1];
     d.workspaceBytes = ws;
-    if (ws)
+    if (ws && select_gqa(p) == GqaKernel::Prefill) {
+      d.buf[4] = {Space::Partials, 0, 0};
+      plan_.partialBytes = std::max(plan_.partialBytes, (ws + kAlign - 1) / kAlign * kAlign);
+    } else if (ws) {
       d.buf[4] = temporary(ws);
+    }
     return LLMI_HIP_OK;
   }
   default:
@@ -1490,7 +1498,7 @@ int Lowering::run() {
     if (int rc = lower(index_))
       return rc;
   }
-  plan_.scratchBytes = (arena_.size() + kAlign - 1) / kAlign * kAlign;
+  plan_.scratchBytes = (arena_.size() + kAlign - 1) / kAlign * kAlign + plan_.partialBytes;
   merge_norm_linears();
   for (const auto &d : plan_.dispatches) {
     for (const Rec &r : d.recs) // op by op, so the records stay in op order
@@ -1510,7 +1518,7 @@ int Lowering::run() {
 }
 
 struct Bases {
-  unsigned char *scratch;
+  unsigned char *scratch, *partials;
   void *const *states;
   const llmi_weight *weights;
   const uint32_t *tokens;
@@ -1525,6 +1533,9 @@ void *resolve(const Bases &b, const Ref &r) {
     return nullptr;
   case Space::Scratch:
     base = b.scratch;
+    break;
+  case Space::Partials:
+    base = b.partials;
     break;
   case Space::Weight:
     base = (unsigned char *)b.weights[r.index].data;
@@ -1673,6 +1684,8 @@ size_t llmi_hip_plan_scratch_bytes(const llmi_hip_plan *plan) {
   return plan ? plan->scratchBytes : 0;
 }
 
+size_t llmi::plan_partial_bytes(const llmi_hip_plan *plan) { return plan->partialBytes; }
+
 void llmi_hip_plan_logits(const llmi_hip_plan *plan, uint64_t *rows, uint64_t *elements) {
   if (rows)
     *rows = plan ? plan->logitRows : 0;
@@ -1703,9 +1716,10 @@ int llmi_hip_plan_execute(const llmi_hip_plan *plan, void *scratch, size_t scrat
                           uint16_t *logits, uint32_t *invalid, void *stream) {
   if (!plan)
     return fail(LLMI_HIP_INVALID_ARGUMENT, "plan: null plan");
-  if (scratch_bytes < plan->scratchBytes || (plan->scratchBytes && !scratch))
+  const uint64_t required = plan->scratchBytes - plan->partialBytes;
+  if (scratch_bytes < required || (required && !scratch))
     return fail(LLMI_HIP_WORKSPACE, "plan: needs a %llu-byte scratch arena",
-                (unsigned long long)plan->scratchBytes);
+                (unsigned long long)required);
   if (state_count != plan->stateCount || (state_count && !states))
     return fail(LLMI_HIP_INVALID_ARGUMENT, "plan: expects %zu state buffers",
                 plan->stateCount);
@@ -1715,7 +1729,7 @@ int llmi_hip_plan_execute(const llmi_hip_plan *plan, void *scratch, size_t scrat
   if (!token_ids || (plan->hasOutput && !logits))
     return fail(LLMI_HIP_INVALID_ARGUMENT, "plan: null token IDs or logits");
   unsigned char *base = static_cast<unsigned char *>(scratch);
-  const Bases b{base, states, plan->weights.data(), token_ids, logits,
+  const Bases b{base, scratch_bytes < plan->scratchBytes ? nullptr : base + required, states, plan->weights.data(), token_ids, logits,
                 invalid ? invalid : reinterpret_cast<uint32_t *>(base + plan->invalidOffset)};
   for (const auto &d : plan->dispatches)
     if (int rc = run_dispatch(d, b, static_cast<hipStream_t>(stream)))

@@ -265,6 +265,37 @@ int session(char **a) {
   return 0;
 }
 
+// model past tokens limit: a step of a two-layer model after `past` rows (in
+// steps of 16) whose new allocations may take up to `limit` bytes each, then a
+// plan of the same step through llmi_hip_model_run.
+int model(char **a) {
+  const uint64_t past = atoi(a[0]), tokens = atoi(a[1]);
+  Model m(past + 2 * tokens);
+  const std::vector<uint32_t> ids(tokens < 16 ? 16 : tokens, 1);
+  for (uint64_t p = 0; p < past; p += 16)
+    if (llmi_hip_model_step(m.session, ids.data(), 16, LLMI_LOGITS_NONE, nullptr, 0, nullptr))
+      return 1;
+  llmi_hip_model_step_result r{};
+  largest = strtoull(a[2], nullptr, 0);
+  launches.clear();
+  printf("status %d\n", llmi_hip_model_step(m.session, ids.data(), tokens, LLMI_LOGITS_NONE,
+                                            nullptr, 0, &r));
+  flush_launches("launches");
+  std::vector<llmi_hip_dispatch> records(llmi_hip_model_dispatches(m.session, nullptr, 0));
+  llmi_hip_model_dispatches(m.session, records.data(), records.size());
+  printf("names");
+  for (const auto &d : records)
+    printf(" %s", d.kernel);
+  printf("\nscratch %llu\ncount %zu\n", (unsigned long long)r.scratch_bytes, r.dispatch_count);
+  llmi_hip_plan *plan = nullptr;
+  if (llmi_hip_model_plan(m.session, tokens, past + tokens, LLMI_LOGITS_NONE, &plan))
+    return 1;
+  printf("run %d\n", llmi_hip_model_run(m.session, plan, ids.data(), nullptr));
+  flush_launches("again");
+  llmi_hip_plan_destroy(plan);
+  return 0;
+}
+
 double half_value(unsigned h) {
   const int e = h >> 10 & 0x1F, f = h & 0x3FF;
   const double m = e == 0x1F ? (f ? NAN : INFINITY)
@@ -307,6 +338,8 @@ int main(int argc, char **argv) {
     return gqa(argv + 2);
   if (command == "session" && argc == 5)
     return session(argv + 2);
+  if (command == "model" && argc == 5)
+    return model(argv + 2);
   if (command == "logits" && argc == 3)
     return logits(argv + 2);
   return 2;

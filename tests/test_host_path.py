@@ -96,3 +96,23 @@ def test_session_step_without_a_decode_workspace_is_refused(host):
     got = dict(host("session", 16411, 1, 1 << 16))
     assert got["status"] == [str(_lib.WORKSPACE)] and got["launches"] == []
     assert got["past"] == ["16411"]
+
+
+def test_model_step_runs_undivided_where_the_partials_find_no_room(host):
+    past, tokens = 640, 300
+    merges = lambda names: sum("refill_merge" in n or "PrefillMerge" in n for n in names)
+    full = dict(host("model", past, tokens, NO_LIMIT))
+    assert full["status"] == full["run"] == ["0"]
+    assert merges(full["launches"]) == merges(full["again"]) == merges(full["names"]) == 1
+    partials = _lib.load().llmi_hip_gqa_workspace_bytes(_lib.GqaParams(tokens, 4, 2, 256, past))
+    partials = (partials + 255) // 256 * 256
+    everything = int(full["scratch"][0])
+    for limit in (everything - 1, everything - partials):
+        got = dict(host("model", past, tokens, limit))
+        assert got["status"] == got["run"] == ["0"]
+        assert merges(got["launches"]) == merges(got["again"]) == merges(got["names"]) == 0
+        assert int(got["scratch"][0]) == everything - partials
+        assert int(got["count"][0]) == len(got["names"]) == len(full["names"]) - 1
+        assert [n for n in full["launches"] if "prefill_merge" not in n] == got["launches"]
+    short = dict(host("model", past, tokens, everything - partials - 1))
+    assert short["status"] == [str(_lib.WORKSPACE)] and short["launches"] == []

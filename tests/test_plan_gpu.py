@@ -18,6 +18,7 @@ import torch
 
 import oracle
 from graph_runner import GraphRunner
+from llminfer_amd import _lib
 from llminfer_amd import graph as G
 from llminfer_amd.plan import ModelSession, random_weights
 from test_plan import TOKENS, oracle_states, run_oracle, tiny_weights
@@ -183,6 +184,55 @@ def test_small_plan_on_the_hot_kernels(gpu):
         print(f"  small plan vs oracle: rel L2 {rel:.3g}, max {np.abs(p - w_).max():.3g}",
               flush=True)
         assert rel <= 0.02 and np.abs(p - w_).max() < 0.05
+
+
+@pytest.mark.parametrize("q_heads", [4, 8])
+def test_prefill_after_a_long_past_is_the_op_by_op_graph(gpu, q_heads):
+    """The second and later turns of a conversation: several rows on 512 and
+    more past rows, whose attention divides its keys (both kernels: two and
+    four query heads a KV head), with one-row steps between."""
+    c = G.Qwen35Config(**{**small_qwen35().__dict__, "q_heads": q_heads})
+    weights = _small_weights(c, 11)
+    rng = np.random.default_rng(12)
+    chunks = [list(rng.integers(0, c.vocabulary, n)) for n in (512, 2, 61, 1, 512, 1, 33)]
+    session, plan_logits, op_logits, states = run_plan_and_ops(c, weights, chunks, True, gpu,
+                                                               capacity=1200)
+    for p, o in zip(plan_logits, op_logits):
+        assert np.array_equal(p.view(np.uint32), o.view(np.uint32))
+    for a, b in zip(session.states, states):
+        assert _same_state(a, b)
+    assert "gqaPrefillMerge" in {d["kernel"] for d in session.plan(2, "last", 1100).dispatches}
+
+
+def test_plan_without_its_partials_runs_undivided(gpu):
+    """An arena that ends before the divided prefill's partials: the attention
+    runs undivided and leaves what lies after the arena alone."""
+    c = small_qwen35()
+    T, past = 61, 700
+    session = ModelSession(c, device_weights(_small_weights(c, 13), gpu), 1024, True, gpu)
+    rng = np.random.default_rng(14)
+    session.step(list(rng.integers(0, c.vocabulary, past)), "none")
+    before = session.states
+    ids = torch.from_numpy(rng.integers(0, c.vocabulary, T).astype(np.int32)).to(gpu)
+    want = session.step(ids.cpu().numpy()).logits
+    plan = session.plan(T, "last", past)
+    need = _lib.load().llmi_hip_gqa_workspace_bytes(
+        _lib.GqaParams(T, c.q_heads, c.kv_heads, c.head_dim, past))
+    least = plan.scratch_bytes - (need + 255) // 256 * 256
+    logits = []
+    for size in (plan.scratch_bytes, least):
+        arena = torch.full((plan.scratch_bytes,), 0xFF, dtype=torch.uint8, device=gpu)
+        states = [t.clone() for t in before]
+        out = torch.empty(1, c.vocabulary, dtype=torch.float16, device=gpu)
+        plan.execute(arena[:size], states, ids, out, None)
+        torch.cuda.synchronize()
+        assert size == plan.scratch_bytes or bool((arena[size:] == 0xFF).all())
+        logits.append(out.float().cpu().numpy())
+    assert np.array_equal(logits[0], want)
+    # the attention's sums in another order, then as against the oracle above
+    assert np.linalg.norm(logits[1] - want) <= 0.02 * np.linalg.norm(want)
+    with pytest.raises(_lib.HipError):
+        plan.execute(arena[:least - 256], before, ids, out, None)
 
 
 def test_session_rejects_bad_steps_and_resets(gpu):
