@@ -556,6 +556,22 @@ def gqa_params(q: torch.Tensor, k_cache: torch.Tensor, past: int) -> _lib.GqaPar
     return _lib.GqaParams(T, hq, k_cache.shape[1], d, past)
 
 
+def _gqa_workspace(lib, p: _lib.GqaParams, device: torch.device) -> tuple:
+    """The attention's workspace and its bytes. A decode step needs it; a
+    prefill that finds no memory for its divided keys' partials runs
+    undivided."""
+    need = lib.llmi_hip_gqa_workspace_bytes(p)
+    if not need:
+        return None, 0
+    try:
+        ws = workspace(need, device)
+    except torch.cuda.OutOfMemoryError:
+        if p.tokens == 1:
+            raise
+        return None, 0
+    return ws, ws.numel()
+
+
 def causal_gqa(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                past: int, out: torch.Tensor | None = None) -> torch.Tensor:
     """CausalGqa over cache rows [0, past+T) (the step's rows already appended)."""
@@ -572,11 +588,9 @@ def causal_gqa(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     _require(out, torch.float16, "out")
     lib = _lib.load()
     p = gqa_params(q, k_cache, past)
-    need = lib.llmi_hip_gqa_workspace_bytes(p)
-    ws = workspace(need, q.device) if need else None
+    ws, nbytes = _gqa_workspace(lib, p, q.device)
     _lib.check(lib.llmi_hip_causal_gqa(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out),
-                                       p, _ptr(ws), ws.numel() if ws is not None else 0,
-                                       _stream()))
+                                       p, _ptr(ws), nbytes, _stream()))
     return out
 
 
@@ -598,11 +612,10 @@ def kv_append_causal_gqa(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     _require(out, torch.float16, "out")
     lib = _lib.load()
     p = gqa_params(q, k_cache, past)
-    need = lib.llmi_hip_gqa_workspace_bytes(p)
-    ws = workspace(need, q.device) if need else None
+    ws, nbytes = _gqa_workspace(lib, p, q.device)
     _lib.check(lib.llmi_hip_kv_append_causal_gqa(
         _ptr(q), _ptr(k), _ptr(v), _ptr(k_cache), _ptr(v_cache), _ptr(out), p, _ptr(ws),
-        ws.numel() if ws is not None else 0, _stream()))
+        nbytes, _stream()))
     return out
 
 
@@ -667,11 +680,10 @@ def bind_gated_attention(q_proj: torch.Tensor, k_proj: torch.Tensor, v_new: torc
         raise ValueError("gated attention shapes do not match the cache")
     lib = _lib.load()
     p = _lib.GqaParams(T, hq, hkv, d, past)
-    need = lib.llmi_hip_gqa_workspace_bytes(p)
-    ws = workspace(need, q_proj.device) if need else None
+    ws, nbytes = _gqa_workspace(lib, p, q_proj.device)
     args = (_ptr(q_proj), _ptr(k_proj), _ptr(v_new), _ptr(q_weight), _ptr(k_weight),
             _ptr(k_cache), _ptr(v_cache), _ptr(out), p, rotary_dim, epsilon, theta, _ptr(ws),
-            ws.numel() if ws is not None else 0, _stream())
+            nbytes, _stream())
     names = kernel_names(_lib.OP_GATED_ATTENTION, p)
     fn = lib.llmi_hip_gated_attention_activated if activated else lib.llmi_hip_gated_attention
     b = Bound(fn, args, "+".join(names))
@@ -873,10 +885,9 @@ def bind_causal_gqa(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         raise ValueError("CausalGqa operands do not match the cache")
     lib = _lib.load()
     p = gqa_params(q, k_cache, past)
-    need = lib.llmi_hip_gqa_workspace_bytes(p)
-    ws = workspace(need, q.device) if need else None
-    args = (_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), p, _ptr(ws),
-            ws.numel() if ws is not None else 0, _stream())
+    ws, nbytes = _gqa_workspace(lib, p, q.device)
+    args = (_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), p, _ptr(ws), nbytes,
+            _stream())
     b = Bound(lib.llmi_hip_causal_gqa, args, kernel_names(_lib.OP_CAUSAL_GQA, p)[0])
     b._keep = ws
     return b
@@ -894,10 +905,9 @@ def bind_kv_append_causal_gqa(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         raise ValueError("KvAppend/CausalGqa operands do not match the cache")
     lib = _lib.load()
     p = gqa_params(q, k_cache, past)
-    need = lib.llmi_hip_gqa_workspace_bytes(p)
-    ws = workspace(need, q.device) if need else None
+    ws, nbytes = _gqa_workspace(lib, p, q.device)
     args = (_ptr(q), _ptr(k), _ptr(v), _ptr(k_cache), _ptr(v_cache), _ptr(out), p, _ptr(ws),
-            ws.numel() if ws is not None else 0, _stream())
+            nbytes, _stream())
     names = kernel_names(_lib.OP_KV_APPEND_CAUSAL_GQA, p)
     b = Bound(lib.llmi_hip_kv_append_causal_gqa, args, "+".join(names))
     b._keep = ws

@@ -7,8 +7,9 @@ import os
 import subprocess
 
 import pytest
+import torch
 
-from llminfer_amd import _lib
+from llminfer_amd import _lib, ops
 from tests.conftest import ROOT
 
 
@@ -116,3 +117,14 @@ def test_model_step_runs_undivided_where_the_partials_find_no_room(host):
         assert [n for n in full["launches"] if "prefill_merge" not in n] == got["launches"]
     short = dict(host("model", past, tokens, everything - partials - 1))
     assert short["status"] == [str(_lib.WORKSPACE)] and short["launches"] == []
+
+
+def test_prefill_takes_no_workspace_where_torch_has_none(monkeypatch):
+    def full(need, device):
+        raise torch.cuda.OutOfMemoryError
+    monkeypatch.setattr(ops, "workspace", full)
+    lib, params = _lib.load(), lambda T, past: _lib.GqaParams(T, 16, 4, 256, past)
+    assert ops._gqa_workspace(lib, params(61, 4096), "cuda") == (None, 0)
+    assert ops._gqa_workspace(lib, params(61, 100), "cuda") == (None, 0)
+    with pytest.raises(torch.cuda.OutOfMemoryError):
+        ops._gqa_workspace(lib, params(1, 4096), "cuda")
