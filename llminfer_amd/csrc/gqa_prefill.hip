@@ -1050,18 +1050,23 @@ hipError_t launch_halves(const GqaShape &s, const uint16_t *q, const uint16_t *k
   return hipGetLastError();
 }
 
-// The key-split kernel once the grid has at least 64 workgroups (below
-// that, as at 128 tokens, the single-wave kernel's shorter prologue wins by
-// ~1 us). LLMI_PREFILL_HALVES=0 selects the single-wave kernel always, =1
-// the key-split one always (for A/B timing). The plain and gated launches
-// take the same choice, so the two stay bit-identical.
-bool use_halves(const GqaShape &s) {
+// LLMI_PREFILL_HALVES=0 selects the single-wave kernel always, =1 the
+// key-split one wherever it runs (for A/B timing): 0, 1, or -1 unset.
+int forced_halves() {
   static const int forced = [] {
     const char *e = getenv("LLMI_PREFILL_HALVES");
     return e && *e ? (*e == '0' ? 0 : 1) : -1;
   }();
-  if (forced >= 0)
-    return forced == 1;
+  return forced;
+}
+
+// The key-split kernel once the grid has at least 64 workgroups (below
+// that, as at 128 tokens, the single-wave kernel's shorter prologue wins by
+// ~1 us). The plain and gated launches take the same choice, so the two stay
+// bit-identical.
+bool use_halves(const GqaShape &s) {
+  if (forced_halves() >= 0)
+    return forced_halves() == 1;
   const unsigned nb = (s.T + BM - 1) / BM, hpairs = s.Hq / s.Hkv / 2;
   return (nb + 1) / 2 * s.Hkv * hpairs >= 64;
 }
@@ -1137,7 +1142,7 @@ SplitPlan split_plan(const GqaShape &s) {
     return p;
   const unsigned G = s.Hq / s.Hkv, nb = (s.T + BM - 1) / BM;
   const unsigned hw = s.D == 256 ? heads_per_wg<256>(G) : heads_per_wg<128>(G);
-  p.halves = s.D == 256 && hw == 4 && nb >= 2;
+  p.halves = s.D == 256 && hw == 4 && (forced_halves() >= 0 ? forced_halves() == 1 : nb >= 2);
   const uint64_t base = p.halves ? (uint64_t)(nb + 1) / 2 * s.Hkv * (G / 2)
                                  : (uint64_t)nb * s.Hkv * (G / hw);
   const unsigned most = s.P / BN / kSplitSteps;

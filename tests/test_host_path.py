@@ -128,3 +128,15 @@ def test_prefill_takes_no_workspace_where_torch_has_none(monkeypatch):
     assert ops._gqa_workspace(lib, params(61, 100), "cuda") == (None, 0)
     with pytest.raises(torch.cuda.OutOfMemoryError):
         ops._gqa_workspace(lib, params(1, 4096), "cuda")
+
+
+@pytest.mark.parametrize("T", [20, 61, 500])
+@pytest.mark.parametrize("past", [0, 4096])
+@pytest.mark.parametrize("forced", ["0", "1"])
+def test_prefill_kernel_switch_holds_for_divided_keys_too(host, T, past, forced):
+    """LLMI_PREFILL_HALVES at the heads that the key-split kernel takes (four a
+    workgroup; a short undivided prefill serves two, by the other kernel)."""
+    got = dict(host("gqa", T, past, 16, 4, 256, 0, env={"LLMI_PREFILL_HALVES": forced}))
+    assert got["status"] == ["0"] and len(got["launches"]) == (2 if past else 1)
+    halves = forced == "1" and (past > 0 or T == 500)
+    assert got["launches"][0] == ("gqa_prefill_halves_kernel" if halves else "gqa_prefill_kernel")
