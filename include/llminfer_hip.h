@@ -352,8 +352,10 @@ LLMI_HIP_API int llmi_hip_kv_append_causal_gqa_noalloc(const uint16_t *q,
  * merge where it divides its keys. Workspace:
  * llmi_hip_gqa_workspace_bytes(p), as for llmi_hip_causal_gqa (the bits are
  * those of that call with as large a workspace).
- * Supported: d 128 or 256, Hq/Hkv 2 or 4 (decode) or <= 4 (prefill),
- * rotary_dim a multiple of 16 up to d; other shapes return UNSUPPORTED. */
+ * Supported: d 128 or 256; decode with Hq/Hkv 2 or 4 and rotary_dim a multiple
+ * of 16 up to d; prefill with Hq/Hkv 1, 2 or 4 (8 too at d 256) and rotary_dim a
+ * multiple of 16 up to 96 at d 128, 224 at d 256. Other shapes return
+ * UNSUPPORTED. */
 LLMI_HIP_API int llmi_hip_gated_attention(const uint16_t *q_proj, const uint16_t *k_proj,
                                           const uint16_t *v_new, const float *q_weight,
                                           const float *k_weight, uint16_t *k_cache,

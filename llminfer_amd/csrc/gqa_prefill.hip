@@ -43,7 +43,8 @@
 //
 // The gated call's query rows are normalised by a launch of their own, into
 // the output (launch_attention_rows): inside these kernels, one or two waves a
-// SIMD, that work took 22 us (333 tokens: 47.5 us with it, 25.5 without).
+// SIMD, that work took 11 us (333 tokens, traced: 45.3 us with it, 34.8 without,
+// 29.0 where the gates are already activated, 20.1 for the attention alone).
 #include "hip_common.hpp"
 #include "kernels.hpp"
 #include "rope_gate.hpp"
@@ -1128,7 +1129,9 @@ hipError_t launch_d(const GqaShape &s, const uint16_t *q, const uint16_t *k,
 // rows: 32.8 us unsplit, 19.7 / 21.6 / 27.0 at 3 / 4 / 6 tiles a split; 512
 // tokens on 500: 31.7 unsplit, 33.8 at 3), so at 511 past rows and fewer
 // nothing is split. At head_dim 256 two blocks of rows and more run as the
-// key-split kernel's pairs.
+// key-split kernel's pairs. A block's keys are divided by a whole number, so a
+// grid of more than half the CUs stays as it is: 1024 tokens on 4096 rows take
+// 99 us in two splits, 1025 tokens 123 in none (head_dim 128: 64 and 89).
 constexpr unsigned kSplitSteps = 4, kSplitWorkgroups = 256;
 static_assert(kSplitSteps >= 3, "a split's first tile is visible to every row of its block");
 
@@ -1207,7 +1210,9 @@ bool prefill_supported(const GqaShape &s) {
 }
 
 bool prefill_gated_supported(const GqaShape &s, unsigned rot) {
-  // (the shapes that the call has always taken)
+  // The shapes that the call has always taken: those whose normalised query
+  // tile and its tables fit a key tile's LDS, where they once lay. At head_dim
+  // 128 rotary widths to 96 and up to four heads, at 256 to 224.
   const unsigned HW = s.D == 256 ? heads_per_wg<256>(s.Hkv ? s.Hq / s.Hkv : 0)
                                  : heads_per_wg<128>(s.Hkv ? s.Hq / s.Hkv : 0);
   const size_t need = (size_t)BM * (s.D + 8) * 2 + BM * 4 + (size_t)s.D * 4 +

@@ -326,13 +326,14 @@ hipError_t launch_copy_half_view(const uint16_t *src, uint16_t *out, const HalfV
 
 hipError_t launch_linear_f16(const uint16_t *in, const uint16_t *w, void *out, const void *aux,
                              const float *bias, const LinearParams &p, hipStream_t stream) {
-  // Up to kF16FewTiles 16 x 16 tiles a tile a workgroup spreads the chains
-  // (8192 columns of 2560 for one row: 17.5 us against 21.9 with four column
-  // tiles a workgroup and 20.4 with 2 x 2; 2560 columns of 9216 for 33 rows:
-  // 55 against 72 and 65). Past that four waves share what a workgroup stages:
-  // four column tiles while there is one row of tiles (248,320 columns: 346 us
-  // against 366 and 404), else 2 x 2 (9216 columns of 2560, 93 rows: 62 us
-  // against 82 with 1 x 4 and 95 with one tile).
+  // Up to kF16FewTiles 16 x 16 tiles, two workgroups a CU, a tile a workgroup
+  // spreads the chains; past that a CU's third one waits for its matrix cores,
+  // and four waves share what a workgroup stages: four column tiles while there
+  // is one row of tiles, else 2 x 2. One tile / 1 x 4 / 2 x 2, us, a width of
+  // 2560: one row of 8192 columns (512 tiles) 18.6 / 23.2 / 21.0, of 9216 (576)
+  // 24.9 / 23.4 / 32.3, of 16384 30.0 / 27.5 / 33.3, of 248,320 369 / 352 / 404;
+  // 33 rows of 2560 columns (480) 17.4 / 22.7 / 20.4, of 4096 (768) 25.4 / 22.8 /
+  // 20.5; 93 rows of 9216 95 / 83 / 60.
   const unsigned rowTiles = (p.tokens + kF16Tile - 1) / kF16Tile;
   const uint64_t tiles = (uint64_t)rowTiles * ((p.rowCount + kF16Tile - 1) / kF16Tile);
   if (tiles <= kF16FewTiles)

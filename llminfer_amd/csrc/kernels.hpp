@@ -186,7 +186,7 @@ bool norm_rope_wide_rows(const RopeShape &s);
 hipError_t launch_norm_rope(const uint16_t *in, const float *w, uint16_t *out,
                             const RopeShape &s, hipStream_t stream);
 // A prefill's rows ahead of its attention: normRope of the queries and of the
-// new keys and the copy of `count` value halves, in one launch where the tile
+// new keys (both normalised, at one theta and rotary width) and the copy of `count` value halves, in one launch where the tile
 // kernel takes both shapes, everything is 16-byte aligned and each input lies
 // apart from the other parts' outputs, else in three: the keys', the values',
 // the queries'.

@@ -506,8 +506,8 @@ hipError_t launch_attention_rows(const uint16_t *q, const float *qw, uint16_t *q
   const uint16_t *krows = kout + (size_t)ks.out_row0 * ks.D;
   if (!apart(k, nk, qout, nqo) || !apart(k, nk, vout, count) || !apart(v, count, qout, nqo) ||
       !apart(v, count, krows, nko) || !apart(q, nq, krows, nko) || !apart(q, nq, vout, count) ||
-      !norm_rope_tiled(qs, q, qout) || !norm_rope_tiled(ks, k, kout) || !qs.norm || !ks.norm ||
-      qs.theta != ks.theta || qs.rot != ks.rot || count % 8 || !aligned16(v) || !aligned16(vout)) {
+      !norm_rope_tiled(qs, q, qout) || !norm_rope_tiled(ks, k, kout) || count % 8 ||
+      !aligned16(v) || !aligned16(vout)) {
     hipError_t e = launch_norm_rope(k, kw, kout, ks, stream);
     if (e == hipSuccess)
       e = launch_cache_append(v, vout, count, 0, stream);

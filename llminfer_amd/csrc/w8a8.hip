@@ -438,7 +438,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemv_split_kernel(
 // Bounds: from a few hundred rows the fp32 work that this order demands, per
 // output and group a conversion (2.3 ns a wave64 operation a SIMD), two
 // products (1.2 each) and an addition (1.5): 36 us for 512 rows of a 2560 ->
-// 9216 projection, where the kernel takes 60; below that the latency of a
+// 9216 projection, where the kernel takes 60 to 71; below that the latency of a
 // step. So waves in flight decide: a tile a workgroup, 64 registers and 37 KB
 // of LDS, four workgroups a CU.
 //
@@ -447,11 +447,14 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemv_split_kernel(
 // buffered; the scales come through registers, requested a step before they
 // are staged. One barrier a step, behind a wait for everything but the last
 // request of scales.
-// Measured (weights rotating past the MALL; 512 rows of 2560 -> 9216, 512 of
-// 9216 -> 2560, 128 of 2560 -> 9216, 13 of 9216 -> 2560):
+// Measured (512 rows of 2560 -> 9216, 512 of 9216 -> 2560, 128 of 2560 ->
+// 9216, 13 of 9216 -> 2560):
 //   through registers and a padded layout      74.4, 73.4, 24.5, 58.1 us
 //   this                                       60.5, 61.1, 19.5, 21.2 us
-// (the fourth ran a kernel of four rows a lane). Not kept: 64 x 32, 32 x 64
+//   traced, uniform random int8 rows           69.8, 69.6, 23.9, 28.0 us
+//   the same, the weights in the MALL          70.4, 70.0, 18.4, 14.5 us
+// (the first row's fourth ran a kernel of four rows a lane; the two traced rows
+// are of another day's card). Not kept: 64 x 32, 32 x 64
 // and 64 x 64 tiles (61 - 65 us at 512 rows with half the loads, but four or
 // two waves a SIMD; 33 and 49 us at 13 rows); three and four buffers (64 - 90
 // us: fewer workgroups a CU); the row scales by DPP broadcast inside the

@@ -184,12 +184,13 @@ def test_prefill_cfg3_every_token(gpu):
 
 # The keys divided over workgroups: from 512 past rows, one block of rows (the
 # single-wave kernel, any head_dim and group) or pairs of blocks (the key-split
-# kernel: even, odd and ragged counts), few splits and many, a ragged last tile.
+# kernel: even, odd and ragged counts), few splits and many, a ragged last tile,
+# two head groups a KV head.
 @pytest.mark.parametrize("shape,T,past", [
     ((16, 4, 256), 2, 512), ((16, 4, 256), 32, 1031), ((16, 4, 256), 33, 777),
     ((16, 4, 256), 70, 1024), ((16, 4, 256), 97, 2000), ((16, 4, 256), 5, 8200),
     ((4, 2, 256), 20, 900), ((16, 4, 128), 45, 1111), ((8, 1, 128), 40, 703),
-    ((8, 8, 128), 33, 600)])
+    ((8, 8, 128), 33, 600), ((8, 1, 256), 19, 640), ((8, 1, 256), 75, 640)])
 def test_prefill_divided_keys(gpu, shape, T, past):
     hq, hkv, d = shape
     print(f"prefill divided shape={shape} T={T} past={past}", flush=True)
