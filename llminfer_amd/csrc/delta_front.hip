@@ -16,7 +16,7 @@
 // sequence) after reading, so no thread races it. Loads and stores are
 // coalesced across the channels of a wave.
 //
-// l2NormF32: one wave per 4 or 8 rows; the rows are staged in LDS with 16-byte
+// l2NormF32: one wave per 4 to 16 rows; the rows are staged in LDS with 16-byte
 // coalesced loads, lane r sums row r in index order (the reference's fma
 // chain), and the fp32 outputs leave as 16-byte stores. Other widths and
 // unaligned buffers take a thread per row.
@@ -41,8 +41,14 @@ constexpr unsigned kMaxKernel = 8;  // filter taps supported (history 7)
 // 128, rows a wave 16 / 8 / 4 in us, l2NormF32 4.1 / 3.2 / 2.8 at 32 rows,
 // 5.0 / 4.2 / 3.9 at 8192, 5.8 / 5.0 / 5.1 at 16384, 7.1 / 7.0 / 7.7 at 32768;
 // gatedRmsNorm 6.8 / 4.6 / 3.5, 7.8 / 5.9 / 5.3, 8.9 / 7.6 / 7.2, 12.1 / 11.5 /
-// 11.6. So four up to kFewRows, eight past it.
+// 11.6. So four up to kFewRows, eight past it. A narrow row leaves a wave's 64
+// lanes without a 16-byte piece each: eight rows up to 64 wide (16384 rows of 64,
+// gatedRmsNorm: 5.4 / 4.6 / 6.0), sixteen up to 32 (131072 rows of 8: 7.8 / 11.1 /
+// 18.0, l2NormF32 4.7 / 6.1 / 9.8).
 constexpr unsigned kFewRows = 16384;
+static unsigned rows_a_wave(unsigned rows, unsigned width) {
+  return width <= 32 ? 16 : width <= 64 || rows > kFewRows ? 8 : 4;
+}
 
 __global__ __launch_bounds__(256) void causal_conv_kernel(
     const uint16_t *__restrict__ in, const uint16_t *__restrict__ w, uint16_t *hist,
@@ -497,15 +503,15 @@ hipError_t launch_l2_norm(const uint16_t *in, float *out, unsigned rows, unsigne
                           float eps, float scale, hipStream_t stream) {
   if (rows == 0 || width == 0)
     return hipSuccess;
-  if (l2_norm_tiled(width, in, out) && rows <= kFewRows)
-    hipLaunchKernelGGL(l2_norm_tile<4>, dim3((rows + 3) / 4), dim3(64), 0, stream, in, out, rows,
-                       width, eps, scale);
-  else if (l2_norm_tiled(width, in, out))
-    hipLaunchKernelGGL(l2_norm_tile<8>, dim3((rows + 7) / 8), dim3(64), 0, stream, in, out, rows,
-                       width, eps, scale);
-  else
+  if (!l2_norm_tiled(width, in, out)) {
     hipLaunchKernelGGL(l2_norm_rows, dim3((rows + 255) / 256), dim3(256), 0, stream, in, out,
                        rows, width, eps, scale);
+    return hipGetLastError();
+  }
+  const unsigned wave = rows_a_wave(rows, width);
+  const auto kernel = wave == 16 ? l2_norm_tile<16> : wave == 8 ? l2_norm_tile<8> : l2_norm_tile<4>;
+  hipLaunchKernelGGL(kernel, dim3((rows + wave - 1) / wave), dim3(64), 0, stream, in, out, rows,
+                     width, eps, scale);
   return hipGetLastError();
 }
 
@@ -517,14 +523,12 @@ template <bool kActivated, bool kQuant>
 static void launch_gated_tile(const uint16_t *in, const void *gate, const float *w, uint16_t *out,
                               int8_t *q, float *scales, unsigned *invalid, unsigned rows,
                               unsigned width, float eps, hipStream_t stream) {
-  if (rows <= kFewRows)
-    hipLaunchKernelGGL((gated_rms_norm_tile<kActivated, kQuant, 4>), dim3((rows + 3) / 4),
-                       dim3(64), 0, stream, in, gate, w, out, rows, width, eps, q, scales,
-                       invalid);
-  else
-    hipLaunchKernelGGL((gated_rms_norm_tile<kActivated, kQuant, 8>), dim3((rows + 7) / 8),
-                       dim3(64), 0, stream, in, gate, w, out, rows, width, eps, q, scales,
-                       invalid);
+  const unsigned wave = rows_a_wave(rows, width);
+  const auto kernel = wave == 16  ? gated_rms_norm_tile<kActivated, kQuant, 16>
+                      : wave == 8 ? gated_rms_norm_tile<kActivated, kQuant, 8>
+                                  : gated_rms_norm_tile<kActivated, kQuant, 4>;
+  hipLaunchKernelGGL(kernel, dim3((rows + wave - 1) / wave), dim3(64), 0, stream, in, gate, w, out,
+                     rows, width, eps, q, scales, invalid);
 }
 
 hipError_t launch_gated_rms_norm(const uint16_t *in, const void *gate, bool activated,

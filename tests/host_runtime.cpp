@@ -23,6 +23,7 @@ std::map<const void *, std::string> &kernels() {
   return m;
 }
 std::vector<std::string> launches;
+std::vector<unsigned> grids; // blocks along x of each
 size_t largest = SIZE_MAX; // allocations above it fail
 hipError_t last = hipSuccess;
 
@@ -62,8 +63,9 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, hipStream_t 
   *g = config.grid, *b = config.block, *lds = config.lds, *s = config.stream;
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **, size_t, hipStream_t) {
+hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3, void **, size_t, hipStream_t) {
   launches.push_back(kernels()[f]);
+  grids.push_back(grid.x);
   return hipSuccess;
 }
 hipError_t hipMalloc(void **p, size_t n) {
@@ -138,6 +140,7 @@ void flush_launches(const char *what) {
     printf(" %s", n.c_str());
   printf("\n");
   launches.clear();
+  grids.clear();
 }
 
 template <typename P> void names(int op, const P &p) {
@@ -145,6 +148,22 @@ template <typename P> void names(int op, const P &p) {
   for (unsigned i = 0, n = llmi_hip_dispatch_count(op, &p); i < n; ++i)
     printf(" %s", llmi_hip_kernel_name(op, &p, i));
   printf("\n");
+}
+
+// rows rows width: the row norms of a DeltaNet layer, and their blocks.
+int rows(char **a) {
+  const unsigned n = atoi(a[0]), width = atoi(a[1]);
+  void *x = aligned_alloc(256, 256); // (not read)
+  auto *u = static_cast<uint16_t *>(x);
+  auto *f = static_cast<float *>(x);
+  printf("status %d", llmi_hip_l2_norm(u, f, L2Params{n, width, 1e-6f, 1.0f}, nullptr));
+  printf(" %d\n", llmi_hip_gated_rms_norm(u, u, f, u, RowParams{n, width, 1e-6f}, nullptr));
+  printf("grids");
+  for (unsigned g : grids)
+    printf(" %u", g);
+  printf("\n");
+  flush_launches("launches");
+  return 0;
 }
 
 // gated T past q_heads kv_heads head_dim rotary place: where the projected
@@ -334,6 +353,8 @@ int main(int argc, char **argv) {
   const std::string command = argc > 1 ? argv[1] : "";
   if (command == "gated" && argc == 9)
     return gated(argv + 2);
+  if (command == "rows" && argc == 4)
+    return rows(argv + 2);
   if (command == "gqa" && argc == 8)
     return gqa(argv + 2);
   if (command == "session" && argc == 5)

@@ -147,7 +147,9 @@ def test_gate_beta_every_fp16_value(gpu):
 # Four rows a wave up to 16384 rows, eight past it: ragged last waves, either
 # side of the rule, and the widest row.
 @pytest.mark.parametrize("rows,width", [(1, 256), (5, 40), (7, 128), (16383, 8), (16384, 8),
-                                        (16385, 8), (16391, 256)])
+                                        (16385, 8), (16391, 256),
+                                        # sixteen, eight and four rows a wave, and past 16384
+                                        (17, 32), (9, 40), (15, 64), (16383, 72), (16385, 72)])
 def test_row_norms_rows_a_wave(gpu, rows, width):
     rng = np.random.default_rng(rows * 3 + width)
     x, g = _f16(rng, (rows, width)), _f16(rng, (rows, width), 2.0)

@@ -140,3 +140,13 @@ def test_prefill_kernel_switch_holds_for_divided_keys_too(host, T, past, forced)
     assert got["status"] == ["0"] and len(got["launches"]) == (2 if past else 1)
     halves = forced == "1" and (past > 0 or T == 500)
     assert got["launches"][0] == ("gqa_prefill_halves_kernel" if halves else "gqa_prefill_kernel")
+
+
+@pytest.mark.parametrize("rows,width,wave", [
+    (100, 8, 16), (131072, 8, 16), (100000, 32, 16), (100, 40, 8), (100000, 64, 8),
+    (16384, 72, 4), (16385, 72, 8), (16384, 256, 4), (100000, 128, 8)])
+def test_row_norms_rows_a_wave(host, rows, width, wave):
+    got = dict(host("rows", rows, width))
+    assert got["status"] == ["0", "0"]
+    assert got["launches"] == ["l2_norm_tile", "gated_rms_norm_tile"]
+    assert got["grids"] == [str(-(-rows // wave))] * 2
