@@ -165,7 +165,7 @@ __global__ __launch_bounds__(256) void causal_conv_k4(
 // A half of a word that was stored whole: the two stores must stay in order.
 typedef uint16_t __attribute__((may_alias)) word_half_t;
 
-// The 4-tap case of several tokens, two channels a lane and eight tokens: as
+// The 4-tap case of seven tokens and more, two channels a lane and eight tokens: as
 // many outputs a lane in half the loads and stores. The estimates of the SiLU
 // first, then the exact values over those that did not settle: about one in
 // 170 does not, so a wave's 16 outputs take one or two exact passes, each lane
@@ -477,9 +477,13 @@ hipError_t launch_causal_conv(const uint16_t *in, const uint16_t *w, uint16_t *h
   if (T == 0 || C == 0)
     return hipSuccess;
   dim3 grid((C + 255) / 256, (T + kConvBlock - 1) / kConvBlock);
-  // Pairs of channels from whole words (a row then starts on a word); one token
-  // keeps a lane a channel, twice the workgroups for its 8192 channels.
-  if (k == 4 && T > 1 && C % 2 == 0 && aligned16(w) &&
+  // Pairs of channels from whole words (a row then starts on a word), from seven
+  // tokens on: fewer keep a lane a channel, in twice the workgroups and without
+  // the pairs' arithmetic for eight tokens. Lane a channel / pairs, us, 8192
+  // channels: 2 tokens 3.4 / 4.5, 4 4.2 / 4.6, 6 4.7 / 4.9, 8 5.3 / 4.8, 16
+  // 7.2 / 4.8.
+  constexpr unsigned kFewTokens = 6;
+  if (k == 4 && T > kFewTokens && C % 2 == 0 && aligned16(w) &&
       (reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(hist) |
        reinterpret_cast<uintptr_t>(out)) % 4 == 0)
     hipLaunchKernelGGL(causal_conv_k4_pairs,

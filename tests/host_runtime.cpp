@@ -166,6 +166,17 @@ int rows(char **a) {
   return 0;
 }
 
+// conv T channels offset: a 4-tap convolution whose output starts `offset`
+// halves past 16-byte alignment.
+int conv(char **a) {
+  const unsigned T = atoi(a[0]), C = atoi(a[1]);
+  auto *u = static_cast<uint16_t *>(aligned_alloc(256, 256)); // (not read)
+  printf("status %d\n", llmi_hip_causal_conv(u, u, u, u + atoi(a[2]), ConvParams{T, C, 4, 1},
+                                             nullptr));
+  flush_launches("launches");
+  return 0;
+}
+
 // gated T past q_heads kv_heads head_dim rotary place: where the projected
 // keys or values lie ("apart", or in an output of the call).
 int gated(char **a) {
@@ -353,6 +364,8 @@ int main(int argc, char **argv) {
   const std::string command = argc > 1 ? argv[1] : "";
   if (command == "gated" && argc == 9)
     return gated(argv + 2);
+  if (command == "conv" && argc == 5)
+    return conv(argv + 2);
   if (command == "rows" && argc == 4)
     return rows(argv + 2);
   if (command == "gqa" && argc == 8)

@@ -50,7 +50,8 @@ def test_causal_conv(gpu, T, C, k, silu):
 # with a lane a channel.
 @pytest.mark.parametrize("T,C,silu,shift", [
     (2, 2, True, 0), (3, 512, True, 0), (4, 510, False, 0), (8, 514, True, 0),
-    (9, 1026, True, 0), (17, 512, True, 0), (9, 511, True, 0), (9, 512, True, 1)])
+    (9, 1026, True, 0), (17, 512, True, 0), (9, 511, True, 0), (9, 512, True, 1),
+    (6, 514, True, 0), (7, 514, True, 0), (7, 2, True, 0)])
 def test_causal_conv_pairs(gpu, T, C, silu, shift):
     rng = np.random.default_rng(T * 37 + C)
     x, w, h = _f16(rng, (T, C), 3.0), _f16(rng, (C, 4), 0.5), _f16(rng, (C, 3))

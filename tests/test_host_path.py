@@ -150,3 +150,12 @@ def test_row_norms_rows_a_wave(host, rows, width, wave):
     assert got["status"] == ["0", "0"]
     assert got["launches"] == ["l2_norm_tile", "gated_rms_norm_tile"]
     assert got["grids"] == [str(-(-rows // wave))] * 2
+
+
+@pytest.mark.parametrize("T,channels,offset,pairs", [
+    (1, 8192, 0, False), (2, 8192, 0, False), (6, 8192, 0, False), (7, 8192, 0, True),
+    (1024, 2, 0, True), (1024, 8191, 0, False), (1024, 8192, 1, False), (1024, 8192, 2, True)])
+def test_convolution_pairs_channels_from_seven_tokens(host, T, channels, offset, pairs):
+    got = dict(host("conv", T, channels, offset))
+    assert got["status"] == ["0"]
+    assert got["launches"] == ["causal_conv_k4_pairs" if pairs else "causal_conv_k4"]
