@@ -1131,7 +1131,13 @@ hipError_t launch_d(const GqaShape &s, const uint16_t *q, const uint16_t *k,
 // nothing is split. At head_dim 256 two blocks of rows and more run as the
 // key-split kernel's pairs. A block's keys are divided by a whole number, so a
 // grid of more than half the CUs stays as it is: 1024 tokens on 4096 rows take
-// 99 us in two splits, 1025 tokens 123 in none (head_dim 128: 64 and 89).
+// 99 us in two splits, 1025 tokens 123 in none (head_dim 128: 64 and 89). In two
+// splits from 64 workgroups on and at few past rows the plain call pays more for
+// the partials than it saves, and the gated one, whose gates then leave the
+// attention kernel, gains (undivided / divided): 500 tokens of 16 / 4 heads of 256
+// on 512 rows 31.6 / 32.9 us plain, 68.6 / 42.6 gated; 128 of 64 / 16 heads 26.2 /
+// 31.1 and 62.6 / 38.0; 500 of 32 / 8 heads of 128 23.7 / 25.1. Both take one rule,
+// so that their bits agree.
 constexpr unsigned kSplitSteps = 4, kSplitWorkgroups = 256;
 static_assert(kSplitSteps >= 3, "a split's first tile is visible to every row of its block");
 
