@@ -556,20 +556,12 @@ def gqa_params(q: torch.Tensor, k_cache: torch.Tensor, past: int) -> _lib.GqaPar
     return _lib.GqaParams(T, hq, k_cache.shape[1], d, past)
 
 
-def _gqa_workspace(lib, p: _lib.GqaParams, device: torch.device) -> tuple:
-    """The attention's workspace and its bytes. A decode step needs it; a
-    prefill that finds no memory for its divided keys' partials runs
-    undivided."""
-    need = lib.llmi_hip_gqa_workspace_bytes(p)
-    if not need:
-        return None, 0
-    try:
-        ws = workspace(need, device)
-    except torch.cuda.OutOfMemoryError:
-        if p.tokens == 1:
-            raise
-        return None, 0
-    return ws, ws.numel()
+def _undivided(p: _lib.GqaParams) -> None:
+    """Where torch has no memory for the attention's workspace (called in its
+    out-of-memory handler): a prefill runs without, its keys undivided; a
+    decode step needs it."""
+    if p.tokens == 1:
+        raise
 
 
 def causal_gqa(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
@@ -588,9 +580,14 @@ def causal_gqa(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     _require(out, torch.float16, "out")
     lib = _lib.load()
     p = gqa_params(q, k_cache, past)
-    ws, nbytes = _gqa_workspace(lib, p, q.device)
+    need = lib.llmi_hip_gqa_workspace_bytes(p)
+    try:
+        ws = workspace(need, q.device) if need else None
+    except torch.cuda.OutOfMemoryError:
+        ws = _undivided(p)
     _lib.check(lib.llmi_hip_causal_gqa(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out),
-                                       p, _ptr(ws), nbytes, _stream()))
+                                       p, _ptr(ws), ws.numel() if ws is not None else 0,
+                                       _stream()))
     return out
 
 
@@ -612,10 +609,14 @@ def kv_append_causal_gqa(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     _require(out, torch.float16, "out")
     lib = _lib.load()
     p = gqa_params(q, k_cache, past)
-    ws, nbytes = _gqa_workspace(lib, p, q.device)
+    need = lib.llmi_hip_gqa_workspace_bytes(p)
+    try:
+        ws = workspace(need, q.device) if need else None
+    except torch.cuda.OutOfMemoryError:
+        ws = _undivided(p)
     _lib.check(lib.llmi_hip_kv_append_causal_gqa(
         _ptr(q), _ptr(k), _ptr(v), _ptr(k_cache), _ptr(v_cache), _ptr(out), p, _ptr(ws),
-        nbytes, _stream()))
+        ws.numel() if ws is not None else 0, _stream()))
     return out
 
 
@@ -680,10 +681,14 @@ def bind_gated_attention(q_proj: torch.Tensor, k_proj: torch.Tensor, v_new: torc
         raise ValueError("gated attention shapes do not match the cache")
     lib = _lib.load()
     p = _lib.GqaParams(T, hq, hkv, d, past)
-    ws, nbytes = _gqa_workspace(lib, p, q_proj.device)
+    need = lib.llmi_hip_gqa_workspace_bytes(p)
+    try:
+        ws = workspace(need, q_proj.device) if need else None
+    except torch.cuda.OutOfMemoryError:
+        ws = _undivided(p)
     args = (_ptr(q_proj), _ptr(k_proj), _ptr(v_new), _ptr(q_weight), _ptr(k_weight),
             _ptr(k_cache), _ptr(v_cache), _ptr(out), p, rotary_dim, epsilon, theta, _ptr(ws),
-            nbytes, _stream())
+            ws.numel() if ws is not None else 0, _stream())
     names = kernel_names(_lib.OP_GATED_ATTENTION, p)
     fn = lib.llmi_hip_gated_attention_activated if activated else lib.llmi_hip_gated_attention
     b = Bound(fn, args, "+".join(names))
@@ -885,9 +890,13 @@ def bind_causal_gqa(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         raise ValueError("CausalGqa operands do not match the cache")
     lib = _lib.load()
     p = gqa_params(q, k_cache, past)
-    ws, nbytes = _gqa_workspace(lib, p, q.device)
-    args = (_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), p, _ptr(ws), nbytes,
-            _stream())
+    need = lib.llmi_hip_gqa_workspace_bytes(p)
+    try:
+        ws = workspace(need, q.device) if need else None
+    except torch.cuda.OutOfMemoryError:
+        ws = _undivided(p)
+    args = (_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), p, _ptr(ws),
+            ws.numel() if ws is not None else 0, _stream())
     b = Bound(lib.llmi_hip_causal_gqa, args, kernel_names(_lib.OP_CAUSAL_GQA, p)[0])
     b._keep = ws
     return b
@@ -905,9 +914,13 @@ def bind_kv_append_causal_gqa(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         raise ValueError("KvAppend/CausalGqa operands do not match the cache")
     lib = _lib.load()
     p = gqa_params(q, k_cache, past)
-    ws, nbytes = _gqa_workspace(lib, p, q.device)
+    need = lib.llmi_hip_gqa_workspace_bytes(p)
+    try:
+        ws = workspace(need, q.device) if need else None
+    except torch.cuda.OutOfMemoryError:
+        ws = _undivided(p)
     args = (_ptr(q), _ptr(k), _ptr(v), _ptr(k_cache), _ptr(v_cache), _ptr(out), p, _ptr(ws),
-            nbytes, _stream())
+            ws.numel() if ws is not None else 0, _stream())
     names = kernel_names(_lib.OP_KV_APPEND_CAUSAL_GQA, p)
     b = Bound(lib.llmi_hip_kv_append_causal_gqa, args, "+".join(names))
     b._keep = ws

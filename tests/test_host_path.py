@@ -122,12 +122,33 @@ def test_model_step_runs_undivided_where_the_partials_find_no_room(host):
 def test_prefill_takes_no_workspace_where_torch_has_none(monkeypatch):
     def full(need, device):
         raise torch.cuda.OutOfMemoryError
+    calls = []
+    lib = _lib.load()
     monkeypatch.setattr(ops, "workspace", full)
-    lib, params = _lib.load(), lambda T, past: _lib.GqaParams(T, 16, 4, 256, past)
-    assert ops._gqa_workspace(lib, params(61, 4096), "cuda") == (None, 0)
-    assert ops._gqa_workspace(lib, params(61, 100), "cuda") == (None, 0)
-    with pytest.raises(torch.cuda.OutOfMemoryError):
-        ops._gqa_workspace(lib, params(1, 4096), "cuda")
+    monkeypatch.setattr(ops, "_require", lambda *a: None)  # (host tensors)
+    monkeypatch.setattr(ops, "_stream", lambda: None)
+
+    class Recorded:
+        llmi_hip_gqa_workspace_bytes = lib.llmi_hip_gqa_workspace_bytes
+        llmi_hip_causal_gqa = llmi_hip_kv_append_causal_gqa = llmi_hip_gated_attention = \
+            staticmethod(lambda *a: calls.append(a[-3:-1]) or _lib.OK)
+    monkeypatch.setattr(_lib, "load", lambda: Recorded)
+    monkeypatch.setattr(ops, "kernel_names", lambda *a: ["attention"])
+    f16 = lambda *s: torch.zeros(s, dtype=torch.float16)
+    cache, w = f16(700, 4, 256), torch.zeros(256)
+    for T in (61, 1):
+        q, k, qp, out = f16(T, 16, 256), f16(T, 4, 256), f16(T, 16, 512), f16(T, 16, 256)
+        for call in (lambda: ops.causal_gqa(q, cache, cache, 600),
+                     lambda: ops.kv_append_causal_gqa(q, k, k, cache, cache, 600),
+                     lambda: ops.gated_attention(qp, k, k, w, w, cache, cache, 600, 64),
+                     lambda: ops.bind_causal_gqa(q, cache, cache, out, 600)(),
+                     lambda: ops.bind_kv_append_causal_gqa(q, k, k, cache, cache, out, 600)()):
+            if T == 1:
+                with pytest.raises(torch.cuda.OutOfMemoryError):
+                    call()
+            else:
+                call()
+    assert calls == [(None, 0)] * 5
 
 
 @pytest.mark.parametrize("T", [20, 61, 500])
